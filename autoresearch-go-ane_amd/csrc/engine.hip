@@ -199,7 +199,12 @@ hipError_t eng_gemm(ane_engine* e, int cls, const half_t* A, int lda, bool at, c
   // (K-major operands, or M-major ones as the weight gradients read them)
   if (!(at && !bt) && ws && bm == 0 && bn == 0) {
     int sp = 1;
-    gemm_pick_split(M, N, K, epi, e->tr.splitk_cap, &bm, &bn, &sp);
+    const ThinTile t = at || bt ? ThinTile() : gemm_pick_thin(M, N, K, epi);
+    if (t.bm && gemm_thin_aligned(g, epi, p)) {
+      if (epi == EPI_STORE_F || epi == EPI_STORE_H) sp = gemm_pick_thin_splits(M, N, K, e->tr.splitk_cap);
+    } else {
+      gemm_pick_split(M, N, K, epi, e->tr.splitk_cap, &bm, &bn, &sp);
+    }
     if (sp > 1) {
       g.splits = sp;
       g.ws = ws;
@@ -689,13 +694,21 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
   TrainBufs& tb = e->tr;
   const bool fused = defer_norm && !train && llama && e->fused_norm && e->ssq_part;
   e->fwd_rr_nparts = 0;
-  // the residual GEMMs' tile fixes how many partials each norm has
-  int res_bm = 0, res_bn = 0;
-  if (fused) {
+  // the residual GEMMs' tile fixes how many partials each norm has: one per
+  // res_cols columns (tile 0 x 0: gemm_run's thin form, 64 columns)
+  int res_bm = 0, res_bn = 0, res_cols = 0;
+  auto res_tile = [&](int K) -> bool {
+    res_bm = res_bn = 0;
+    if (gemm_pick_thin(T, D, K, EPI_RESID_NORM).bm && D / 64 <= kRrMaxParts) {
+      res_cols = 64;
+      return true;
+    }
     gemm_pick_tile(T, D, H, EPI_RESID_NORM, &res_bm, &res_bn);
-    if (!res_bn || D / res_bn > kRrMaxParts)
-      return eng_fail(e, ANE_ERR_ARG, "storiesane forward: no residual tile for dim=%d", D);
-  }
+    res_cols = res_bn;
+    return res_bn && D / res_bn <= kRrMaxParts;
+  };
+  if (fused && (!res_tile(D) || !res_tile(H)))
+    return eng_fail(e, ANE_ERR_ARG, "storiesane forward: no residual tile for dim=%d", D);
   // RR epilogue parameters over the current partials
   auto rr = [&](EpiParams& p, int nparts) {
     p.rr_part = e->ssq_part; p.rr_ld = T; p.rr_nparts = nparts; p.rr_dim = D;
@@ -783,8 +796,9 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
       if (!llama) { p.alpha_ptr = P + e->pm.resid + l; p.X0 = e->x0; p.beta_ptr = P + e->pm.x0l + l; }
       if (fused) {
         p.C2 = A.xn2; p.ldc2 = D; p.gain = P + o.g_ffn; p.ssq_part = e->ssq_part; p.ssq_ld = T;
+        (void)res_tile(D);
         HIPCHK(op, eng_gemm(e, 1, A.att, D, false, s.wo, D, false, T, D, D, EPI_RESID_NORM, p, res_bm, res_bn));
-        nparts = D / res_bn;
+        nparts = D / res_cols;
       } else {
         HIPCHK(op, eng_gemm(e, 1, A.att, D, false, s.wo, D, false, T, D, D, EPI_RESID, p));
       }
@@ -827,10 +841,11 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
         p.C2 = A.xn; p.ldc2 = D; p.gain = P + (l + 1 < L ? e->pm.L[l + 1].g_att : e->pm.g_final);
         p.ssq_part = e->ssq_part; p.ssq_ld = T;
         // streams the next layer's Wq|Wk|Wv (the classifier's come by a prefetch launch)
+        (void)res_tile(H);
         const void* pf2 = e->gemm_selfpf && l + 1 < L ? (const void*)e->ls[l + 1].wqkv : nullptr;
         HIPCHK(op, eng_gemm(e, 3, A.gate, H, false, s.w2, H, false, T, D, H, EPI_RESID_NORM, p, res_bm, res_bn, false,
                             pf2, (size_t)3 * D * D * sizeof(half_t)));
-        nparts = D / res_bn;
+        nparts = D / res_cols;
       } else {
         HIPCHK(op, eng_gemm(e, 3, A.gate, H, false, s.w2, H, false, T, D, H, EPI_RESID, p));
       }

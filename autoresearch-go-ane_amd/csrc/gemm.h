@@ -129,6 +129,19 @@ hipError_t gemm_run(const GemmArgs& g, int epi, const EpiParams& e, hipStream_t 
 // ws_cap = workspace floats available (splits * M * N must fit).
 void gemm_pick_split(int M, int N, int K, int epi, size_t ws_cap, int* bm, int* bn, int* splits);
 
+// The forms of gemm_thin_kernel (gemm_thin.h), for outputs too small to fill
+// the chip: tile, waves that share its K, LDS stages per wave; bm 0 = none.
+struct ThinTile {
+  int bm = 0, bn = 0, ks = 0, dep = 0;
+};
+// The form gemm_run() takes for a K-major GEMM of this shape when no tile is
+// forced (and its operands are 16-byte aligned); bm = 0: another kernel.
+ThinTile gemm_pick_thin(int M, int N, int K, int epi);
+// Split count for such a GEMM with a very long K (1: none).
+int gemm_pick_thin_splits(int M, int N, int K, size_t ws_cap);
+bool gemm_thin_aligned(const GemmArgs& g, int epi, const EpiParams& e);
+hipError_t gemm_thin_run(const ThinTile& t, const GemmArgs& g, int epi, const EpiParams& e, hipStream_t stream);
+
 // Tile the heuristic picks; nonzero *bm / *bn on entry are kept as
 // constraints (set both to 0 for a free choice).  0 = no tile fits.
 void gemm_pick_tile(int M, int N, int K, int epi, int* bm, int* bn);

@@ -163,20 +163,30 @@ hipError_t gemm_run(const GemmArgs& g, int epi, const EpiParams& e, hipStream_t 
     if ((g.a_t && !g.b_t) || g.grp || !g.ws || (g.K % (g.splits * BK)) != 0 || (ns != 0 && ns != 2) ||
         (epi != EPI_STORE_F && epi != EPI_STORE_H && epi != EPI_STORE_W13) || (g.N % 4) != 0)
       return hipErrorInvalidValue;
-    if (bm == 0 || bn == 0) gemm_pick_tile(g.M, g.N, g.K, epi, &bm, &bn);
-    if (bm == 0 || bn == 0 || (g.M % bm) || (g.N % bn)) return hipErrorInvalidValue;
-    if (nw == 0) nw = (bm == 256 && bn == 256) ? 8 : 4;
-    if (nw != 4 && !(nw == 8 && bm == 256 && bn == 256)) return hipErrorInvalidValue;
     EpiParams pw;  // fp32 partials, ws[s][M][N]
     pw.C = g.ws;
     pw.ldc = g.N;
-    hipError_t r = g.a_t   ? launch<true, true, EPI_STORE_F>(g, pw, s, bm, bn, nw, 2)
+    const ThinTile t = bm || bn || nw || ns ? ThinTile() : gemm_pick_thin(g.M, g.N, g.K, EPI_STORE_F);
+    const bool thin = t.bm && gemm_thin_aligned(g, EPI_STORE_F, pw);
+    if (!thin) {
+      if (bm == 0 || bn == 0) gemm_pick_tile(g.M, g.N, g.K, epi, &bm, &bn);
+      if (bm == 0 || bn == 0 || (g.M % bm) || (g.N % bn)) return hipErrorInvalidValue;
+      if (nw == 0) nw = (bm == 256 && bn == 256) ? 8 : 4;
+      if (nw != 4 && !(nw == 8 && bm == 256 && bn == 256)) return hipErrorInvalidValue;
+    }
+    hipError_t r = thin    ? gemm_thin_run(t, g, EPI_STORE_F, pw, s)
+                   : g.a_t   ? launch<true, true, EPI_STORE_F>(g, pw, s, bm, bn, nw, 2)
                    : g.b_t ? launch<false, true, EPI_STORE_F>(g, pw, s, bm, bn, nw, 2)
                            : launch<false, false, EPI_STORE_F>(g, pw, s, bm, bn, nw, 2);
     if (r != hipSuccess) return r;
     if (epi == EPI_STORE_F) return splitk_reduce<EPI_STORE_F>(g, e, s);
     if (epi == EPI_STORE_H) return splitk_reduce<EPI_STORE_H>(g, e, s);
     return splitk_reduce<EPI_STORE_W13>(g, e, s);
+  }
+  if (!bm && !bn && !nw && !ns && !g.a_t && !g.b_t) {
+    const ThinTile t = gemm_pick_thin(g.M, g.N, g.K, epi);
+    if (t.bm && gemm_thin_aligned(g, epi, e)) return gemm_thin_run(t, g, epi, e, s);
+    if (t.bm && epi == EPI_RESID_NORM) bm = bn = 64;  // the partials its caller counts on are per 64 columns
   }
   if (bm == 0 || bn == 0) gemm_pick_tile(g.M, g.N, g.K, epi, &bm, &bn);
   if (bm == 0 || bn == 0 || (g.M % bm) || (g.N % bn)) return hipErrorInvalidValue;
