@@ -714,6 +714,14 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
     p.rr_part = e->ssq_part; p.rr_ld = T; p.rr_nparts = nparts; p.rr_dim = D;
   };
   int nparts = 1;
+  // a GEMM that runs as gemm_thin_kernel requests its weights whole at its
+  // start: nothing is streamed ahead of it
+  auto ahead = [&](int N, int K, int epi, size_t bytes) { return gemm_pick_thin(T, N, K, epi).bm ? (size_t)0 : bytes; };
+  const size_t qkv_ahead = ahead(3 * D, D, fused ? EPI_STORE_H_RR : EPI_STORE_H, (size_t)3 * D * D * sizeof(half_t));
+  const size_t wo_ahead = ahead(D, D, fused ? EPI_RESID_NORM : EPI_RESID, (size_t)D * D * sizeof(half_t));
+  const size_t ffn_ahead =  // W1|W3, W2
+      ahead(llama ? 2 * H : H, D, fused ? EPI_SWIGLU_RR : llama ? EPI_SWIGLU : EPI_RELU2,
+            ((size_t)(llama ? 2 : 1) * H * D + (size_t)D * H) * sizeof(half_t));
 
   float* x_first = train ? tb.L[0].xin : e->x;
   // a training forward behind an asynchronous update: each part starts once
@@ -723,7 +731,7 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
   if (llama && fused) {
     prof_begin(e, 7);
     HIPCHK(op, embed_xg(x_first, e->xh, e->ssq_part, P + e->pm.embed, e->tok, P + e->pm.L[0].g_att, T, D, V, st,
-                        e->ls[0].wqkv, (size_t)3 * D * D * sizeof(half_t)));
+                        e->ls[0].wqkv, qkv_ahead));
     prof_end(e, 0, (double)T * D * 10);
   } else if (llama) {
     prof_begin(e, 7);
@@ -757,7 +765,7 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
       // the caches (prefetch_slice): QKV here, Wo in attention, W1|W3 + W2 in
       // the FFN norm, the classifier in the final norm
       HIPCHK(op, rmsnorm_f16(A.xn, A.xin, nullptr, nullptr, llama ? P + o.g_att : nullptr, T, D, st, s.wqkv,
-                             (size_t)3 * D * D * sizeof(half_t)));
+                             qkv_ahead));
       prof_end(e, 0, (double)T * D * 6);
     }
     if (fused && l > 0 && e->fused_pf && !e->gemm_selfpf) {
@@ -781,7 +789,7 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
       a.nseq = nseq; a.S = S; a.NH = NH;
       a.qknorm = llama ? 0 : 1;
       a.scale = 0.125f;
-      a.pf = s.wo; a.pf_bytes = (size_t)D * D * sizeof(half_t);
+      a.pf = s.wo; a.pf_bytes = wo_ahead;
       if (o.ve_embed >= 0) {
         a.ve_x = A.xin; a.ve_gate = P + o.ve_gate; a.ve_embed = P + o.ve_embed; a.tokens = e->tok; a.vocab = V;
       }
@@ -806,7 +814,7 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
     if (!fused) {
       prof_begin(e, 6);
       HIPCHK(op, rmsnorm_f16(A.xn2, A.x2, nullptr, nullptr, llama ? P + o.g_ffn : nullptr, T, D, st, s.w13,
-                             ((size_t)(llama ? 2 : 1) * H * D + (size_t)D * H) * sizeof(half_t)));  // W1|W3, W2
+                             ffn_ahead));
       prof_end(e, 0, (double)T * D * 6);
     }
     {
@@ -842,7 +850,7 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
         p.ssq_part = e->ssq_part; p.ssq_ld = T;
         // streams the next layer's Wq|Wk|Wv (the classifier's come by a prefetch launch)
         (void)res_tile(H);
-        const void* pf2 = e->gemm_selfpf && l + 1 < L ? (const void*)e->ls[l + 1].wqkv : nullptr;
+        const void* pf2 = e->gemm_selfpf && qkv_ahead && l + 1 < L ? (const void*)e->ls[l + 1].wqkv : nullptr;
         HIPCHK(op, eng_gemm(e, 3, A.gate, H, false, s.w2, H, false, T, D, H, EPI_RESID_NORM, p, res_bm, res_bn, false,
                             pf2, (size_t)3 * D * D * sizeof(half_t)));
         nparts = D / res_cols;

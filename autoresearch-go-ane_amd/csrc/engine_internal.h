@@ -96,6 +96,7 @@ struct TrainBufs {
   // stream while the main stream's next norms write other partials
   float* dgain_parts = nullptr;
   double* dot_part = nullptr;
+  double* lam_parts = nullptr;  // nanochat: [2 L][nblocks][2], the lambda gradients' partials of each layer's two norms
   double* sumsq = nullptr;
   double* sumsq_part = nullptr;
 };

@@ -139,7 +139,8 @@ int ensure_train(ane_engine* e, const char* op) {
   const size_t nblk = (size_t)norm_bwd_blocks((int)T);
   HIPCHK(op, dalloc(e, &tb.dgain_part, nblk * D));
   if (llama) HIPCHK(op, dalloc(e, &tb.dgain_parts, 2 * (size_t)c.layers * nblk * D));
-  HIPCHK(op, dalloc(e, &tb.dot_part, (nblk > 256 ? nblk : 256) * 2));
+  HIPCHK(op, dalloc(e, &tb.dot_part, 256 * 2));
+  if (!llama) HIPCHK(op, dalloc(e, &tb.lam_parts, 2 * (size_t)c.layers * nblk * 2));
   HIPCHK(op, dalloc(e, &tb.sumsq, 1));
   HIPCHK(op, dalloc(e, &tb.sumsq_part, kSumsqBlocks));
   for (hipEvent_t& ev : e->step_ev) HIPCHK(op, hipEventCreate(&ev));
@@ -241,6 +242,7 @@ int backward_body(ane_engine* e, int nseq, bool async) {
   // dcur_h(l) is the dY that enters layer l from above
   auto by_parity = [&](half_t* a, half_t* b, int l) { return async && (l & 1) ? b : a; };
   auto dcur_h_of = [&](int l) { return by_parity(tb.dcur_h, tb.dcur_h2, l); };
+  auto lpart = [&](int i) { return tb.lam_parts + (size_t)i * nblk * 2; };
   auto gpart = [&](int i) { return tb.dgain_parts + (size_t)i * nblk * D; };
   // llama2, first backward of an accumulation window: every gradient writer
   // (the dW GEMMs, the classifier's gEmbed GEMM, the gain reductions)
@@ -258,8 +260,11 @@ int backward_body(ane_engine* e, int nseq, bool async) {
   // meet each B panel at once and a 64x64-tile GEMM pays ~10 us (W1|W3 dX
   // and dW at B16).  A prefetch issued a few kernels earlier does not help:
   // the data in between evicts it.
+  // Few tokens: the dX GEMMs run as gemm_thin_kernel, which requests its
+  // operands whole, and the saved activations are still in the caches.
+  const bool bwd_ahead = e->bwd_prefetch && !gemm_pick_thin(T, D, KH, EPI_STORE_F).bm;
   auto prefetch = [&](hipStream_t s, std::initializer_list<std::pair<const void*, size_t>> regions) -> hipError_t {
-    if (!e->bwd_prefetch) return hipSuccess;
+    if (!bwd_ahead) return hipSuccess;
     PrefetchList pl;
     for (const auto& r : regions) pl.add(r.first, r.second);
     return prefetch_list(pl, s);
@@ -391,7 +396,7 @@ int backward_body(ane_engine* e, int nseq, bool async) {
       if (llama) {
         a.gain = P + o.g_ffn; a.dgain_part = gpart(2 * l);
       } else {
-        a.lam_x = A.x2; a.lam_x0 = e->x0; a.lam_part = tb.dot_part; a.gx0 = tb.gx0; a.xl_p = xl_p;
+        a.lam_x = A.x2; a.lam_x0 = e->x0; a.lam_part = lpart(2 * l); a.gx0 = tb.gx0; a.xl_p = xl_p;
       }
       HIPCHK(op, norm_bwd(a, st));
       if (async) HIPCHK(op, stream_after(e, ds, st));  // dx2_h and the FFN gain partials written
@@ -400,8 +405,7 @@ int backward_body(ane_engine* e, int nseq, bool async) {
         phase_begin(e, PH_RMS_DW, ds);
         HIPCHK(op, reduce_partials_add(G + o.g_ffn, gpart(2 * l), nblk, D, ds, fresh));
         phase_end(e, ds);
-      } else
-        HIPCHK(op, reduce_dots_add(G + pm.resid + l, G + pm.x0l + l, tb.dot_part, nblk, 1.f, st));
+      }
     }
     // attention (backwardAttentionCPU, ane/train_full.go:644-675)
     {
@@ -482,7 +486,7 @@ int backward_body(ane_engine* e, int nseq, bool async) {
       if (llama) {
         a.gain = P + o.g_att; a.dgain_part = gpart(2 * l + 1);
       } else {
-        a.lam_x = A.xin; a.lam_x0 = e->x0; a.lam_part = tb.dot_part; a.gx0 = tb.gx0; a.xl_p = xl_p;
+        a.lam_x = A.xin; a.lam_x0 = e->x0; a.lam_part = lpart(2 * l + 1); a.gx0 = tb.gx0; a.xl_p = xl_p;
         if (o.ve_embed >= 0) a.ve_dx = tb.ve_dx;
         if (l == L / 2) a.addend2 = tb.ginj;  // ane/train_full.go:784-787
       }
@@ -493,13 +497,14 @@ int backward_body(ane_engine* e, int nseq, bool async) {
         phase_begin(e, PH_RMS_DW);
         HIPCHK(op, reduce_partials_add(G + o.g_att, gpart(2 * l + 1), nblk, D, st, fresh));
         phase_end(e);
-      } else
-        HIPCHK(op, reduce_dots_add(G + pm.resid + l, G + pm.x0l + l, tb.dot_part, nblk, 1.f, st));
+      }
     }
   }
   // every dW launch is done before the embedding side (embed_bwd adds into
   // the embedding gradient the classifier's dW GEMM wrote)
   if (async) HIPCHK(op, stream_after(e, st, ds));
+
+  if (!llama) HIPCHK(op, reduce_lams_add(G + pm.resid, G + pm.x0l, tb.lam_parts, nblk, L, st));
 
   // ---- embedding side ---------------------------------------------------------
   if (!llama) {

@@ -4,7 +4,7 @@
 
 namespace ane {
 
-constexpr int kNormBwdRows = 8;  // rows per block of norm_bwd (4 waves x 2 rows)
+constexpr int kNormBwdRows = 8;  // rows per block of norm_bwd (a wave each)
 
 // out = alpha * addend + addend2 + RMSNorm-backward(dy; x, gain) (+ ve_dx on
 // channels 0..11), fp32 and optionally fp16.  Gain-free form:
@@ -40,6 +40,8 @@ inline int norm_bwd_blocks(int T) { return (T + kNormBwdRows - 1) / kNormBwdRows
 // (overwrite: dst[i] = the sum, the first gradient of an accumulation window)
 hipError_t reduce_partials_add(float* dst, const float* part, int nblocks, int n, hipStream_t s,
                                bool overwrite = false);
+// parts [2 layers][nblocks][2]: dr[l] and dx[l] += the sums of parts 2 l and 2 l + 1
+hipError_t reduce_lams_add(float* dr, float* dx, const double* parts, int nblocks, int layers, hipStream_t s);
 // dst[k] += (float)(sign * sum over blocks of part[b][k])  for k < 2 (lambda grads)
 hipError_t reduce_dots_add(float* dst0, float* dst1, const double* part, int nblocks, float sign, hipStream_t s);
 

@@ -10,113 +10,108 @@ namespace {
 
 constexpr int kMaxVec = 4;  // D <= 1024: float4 groups per lane
 
-__global__ __launch_bounds__(256) void norm_bwd_kernel(NormBwdArgs a) {
-  __shared__ float gsh[4][1024];
-  __shared__ double lsh[4][2];
+// The general form: one wave per row, kNormBwdRows waves per block.  Every
+// load of the row (dy, x, and whichever of the gain, the two addends, x0 and
+// the x0 gradient the call has) is issued before its two reductions, so a
+// row costs one memory round trip; lam_x is x itself in every call that has
+// it and then is not read again.  (4 waves of two rows each, the addends
+// loaded after the reductions: 13.3 us at 256 tokens; this: 7.2.)
+__global__ __launch_bounds__(64 * kNormBwdRows) void norm_bwd_kernel(NormBwdArgs a) {
+  __shared__ float gsh[kNormBwdRows][1024];
+  __shared__ double lsh[kNormBwdRows][2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int D = a.D, nv = D / 4;
+  const int t = blockIdx.x * kNormBwdRows + wave;
+  const bool row_ok = t < a.T;
+  const size_t ro = (size_t)min(t, a.T - 1) * D;  // a row past T (last block) reads row T - 1, stores nothing
   const float alpha = a.alpha_p ? *a.alpha_p : a.alpha;
   const float xl = a.xl_p ? *a.xl_p : 0.f;
-  float4 dg[kMaxVec];
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 dy[kMaxVec], xv[kMaxVec], gv[kMaxVec], ad[kMaxVec], x0[kMaxVec], gx[kMaxVec], a2[kMaxVec];
 #pragma unroll
-  for (int k = 0; k < kMaxVec; k++) dg[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-  double la = 0.0, lb = 0.0;
-  for (int rr = 0; rr < kNormBwdRows / 4; rr++) {
-    const int t = blockIdx.x * kNormBwdRows + wave * (kNormBwdRows / 4) + rr;
-    if (t >= a.T) break;
-    const size_t ro = (size_t)t * D;
-    float4 dy[kMaxVec], xv[kMaxVec], gv[kMaxVec];
-    float ss = 0.f, dot = 0.f;
-#pragma unroll
-    for (int k = 0; k < kMaxVec; k++) {
-      const int i = lane + 64 * k;
-      if (i < nv) {
-        dy[k] = reinterpret_cast<const float4*>(a.dy + ro)[i];
-        xv[k] = reinterpret_cast<const float4*>(a.x + ro)[i];
-        gv[k] = a.gain ? reinterpret_cast<const float4*>(a.gain)[i] : make_float4(1.f, 1.f, 1.f, 1.f);
-        ss += xv[k].x * xv[k].x + xv[k].y * xv[k].y + xv[k].z * xv[k].z + xv[k].w * xv[k].w;
-        dot += dy[k].x * xv[k].x * gv[k].x + dy[k].y * xv[k].y * gv[k].y + dy[k].z * xv[k].z * gv[k].z +
-               dy[k].w * xv[k].w * gv[k].w;
-      }
+  for (int k = 0; k < kMaxVec; k++) {
+    gv[k] = make_float4(1.f, 1.f, 1.f, 1.f);
+    dy[k] = xv[k] = ad[k] = x0[k] = gx[k] = a2[k] = zero;
+    if (64 * k >= nv) continue;  // uniform; lanes past nv read a valid group, their values unused
+    const int i = min(lane + 64 * k, nv - 1);
+    dy[k] = reinterpret_cast<const float4*>(a.dy + ro)[i];
+    xv[k] = reinterpret_cast<const float4*>(a.x + ro)[i];
+    if (a.gain) gv[k] = reinterpret_cast<const float4*>(a.gain)[i];
+    if (a.addend) {
+      ad[k] = reinterpret_cast<const float4*>(a.addend + ro)[i];
+      if (a.lam_x0) x0[k] = reinterpret_cast<const float4*>(a.lam_x0 + ro)[i];
+      if (a.gx0) gx[k] = reinterpret_cast<const float4*>(a.gx0 + ro)[i];
     }
-    ss = wave_sum(ss);
-    dot = wave_sum(dot);
-    const float rrms = 1.0f / sqrtf(ss / (float)D + 1e-5f);
-    const float c = dot * rrms * rrms / (float)D;  // both forms: dx = (dy - x*c) * rrms * gain
-    float pa = 0.f, pb = 0.f;
-#pragma unroll
-    for (int k = 0; k < kMaxVec; k++) {
-      const int i = lane + 64 * k;
-      if (i >= nv) continue;
-      float o[4] = {(dy[k].x - xv[k].x * c) * rrms * gv[k].x, (dy[k].y - xv[k].y * c) * rrms * gv[k].y,
-                    (dy[k].z - xv[k].z * c) * rrms * gv[k].z, (dy[k].w - xv[k].w * c) * rrms * gv[k].w};
-      if (a.dgain_part) {
-        dg[k].x += dy[k].x * xv[k].x * rrms;
-        dg[k].y += dy[k].y * xv[k].y * rrms;
-        dg[k].z += dy[k].z * xv[k].z * rrms;
-        dg[k].w += dy[k].w * xv[k].w * rrms;
-      }
-      if (a.addend) {
-        const float4 ad = reinterpret_cast<const float4*>(a.addend + ro)[i];
-        const float av[4] = {ad.x, ad.y, ad.z, ad.w};
-#pragma unroll
-        for (int u = 0; u < 4; u++) o[u] += alpha * av[u];
-        if (a.lam_x) {
-          const float4 lx = reinterpret_cast<const float4*>(a.lam_x + ro)[i];
-          pa += av[0] * lx.x + av[1] * lx.y + av[2] * lx.z + av[3] * lx.w;
-        }
-        if (a.lam_x0) {
-          const float4 lx = reinterpret_cast<const float4*>(a.lam_x0 + ro)[i];
-          pb += av[0] * lx.x + av[1] * lx.y + av[2] * lx.z + av[3] * lx.w;
-        }
-        if (a.gx0) {
-          float4* gp = reinterpret_cast<float4*>(a.gx0 + ro) + i;
-          float4 gg = *gp;
-          gg.x += xl * av[0]; gg.y += xl * av[1]; gg.z += xl * av[2]; gg.w += xl * av[3];
-          *gp = gg;
-        }
-      }
-      if (a.addend2) {
-        const float4 ad = reinterpret_cast<const float4*>(a.addend2 + ro)[i];
-        o[0] += ad.x; o[1] += ad.y; o[2] += ad.z; o[3] += ad.w;
-      }
-      if (a.ve_dx && i < 3) {  // channels 0..11 = float4 groups 0..2
-#pragma unroll
-        for (int u = 0; u < 4; u++) o[u] += a.ve_dx[(size_t)t * 12 + 4 * i + u];
-      }
-      reinterpret_cast<float4*>(a.out + ro)[i] = make_float4(o[0], o[1], o[2], o[3]);
-      if (a.out_h) {
-        half4 hv;
-#pragma unroll
-        for (int u = 0; u < 4; u++) hv[u] = (half_t)o[u];
-        reinterpret_cast<half4*>(a.out_h + ro)[i] = hv;
-      }
-    }
-    la += (double)pa;
-    lb += (double)pb;
+    if (a.addend2) a2[k] = reinterpret_cast<const float4*>(a.addend2 + ro)[i];
   }
-  if (a.dgain_part) {
+  float4 vd = zero;  // channels 0..11 = float4 groups 0..2
+  if (a.ve_dx && lane < 3) vd = reinterpret_cast<const float4*>(a.ve_dx + (size_t)min(t, a.T - 1) * 12)[lane];
+  float ss = 0.f, dot = 0.f, pa = 0.f, pb = 0.f;
 #pragma unroll
-    for (int k = 0; k < kMaxVec; k++) {
-      const int i = lane + 64 * k;
-      if (i < nv) {
-        gsh[wave][4 * i] = dg[k].x; gsh[wave][4 * i + 1] = dg[k].y;
-        gsh[wave][4 * i + 2] = dg[k].z; gsh[wave][4 * i + 3] = dg[k].w;
+  for (int k = 0; k < kMaxVec; k++) {
+    if (64 * k < nv && lane + 64 * k < nv) {
+      ss += xv[k].x * xv[k].x + xv[k].y * xv[k].y + xv[k].z * xv[k].z + xv[k].w * xv[k].w;
+      dot += dy[k].x * xv[k].x * gv[k].x + dy[k].y * xv[k].y * gv[k].y + dy[k].z * xv[k].z * gv[k].z +
+             dy[k].w * xv[k].w * gv[k].w;
+      if (a.lam_part) {
+        float4 lx = xv[k];
+        if (a.lam_x != a.x) lx = a.lam_x ? reinterpret_cast<const float4*>(a.lam_x + ro)[lane + 64 * k] : zero;
+        pa += ad[k].x * lx.x + ad[k].y * lx.y + ad[k].z * lx.z + ad[k].w * lx.w;
+        pb += ad[k].x * x0[k].x + ad[k].y * x0[k].y + ad[k].z * x0[k].z + ad[k].w * x0[k].w;
       }
+    }
+  }
+  ss = wave_sum_dpp(ss);
+  dot = wave_sum_dpp(dot);
+  const float rrms = 1.0f / sqrtf(ss / (float)D + 1e-5f);
+  const float c = dot * rrms * rrms / (float)D;  // both forms: dx = (dy - x*c) * rrms * gain
+#pragma unroll
+  for (int k = 0; k < kMaxVec; k++) {
+    const int i = lane + 64 * k;
+    if (64 * k >= nv || i >= nv) continue;
+    if (a.dgain_part) {
+      gsh[wave][4 * i] = row_ok ? dy[k].x * xv[k].x * rrms : 0.f;
+      gsh[wave][4 * i + 1] = row_ok ? dy[k].y * xv[k].y * rrms : 0.f;
+      gsh[wave][4 * i + 2] = row_ok ? dy[k].z * xv[k].z * rrms : 0.f;
+      gsh[wave][4 * i + 3] = row_ok ? dy[k].w * xv[k].w * rrms : 0.f;
+    }
+    if (!row_ok) continue;
+    float o[4] = {(dy[k].x - xv[k].x * c) * rrms * gv[k].x, (dy[k].y - xv[k].y * c) * rrms * gv[k].y,
+                  (dy[k].z - xv[k].z * c) * rrms * gv[k].z, (dy[k].w - xv[k].w * c) * rrms * gv[k].w};
+    if (a.addend) {
+      o[0] += alpha * ad[k].x; o[1] += alpha * ad[k].y; o[2] += alpha * ad[k].z; o[3] += alpha * ad[k].w;
+      if (a.gx0)
+        reinterpret_cast<float4*>(a.gx0 + ro)[i] = make_float4(gx[k].x + xl * ad[k].x, gx[k].y + xl * ad[k].y,
+                                                               gx[k].z + xl * ad[k].z, gx[k].w + xl * ad[k].w);
+    }
+    if (a.addend2) { o[0] += a2[k].x; o[1] += a2[k].y; o[2] += a2[k].z; o[3] += a2[k].w; }
+    if (k == 0 && a.ve_dx && lane < 3) { o[0] += vd.x; o[1] += vd.y; o[2] += vd.z; o[3] += vd.w; }
+    reinterpret_cast<float4*>(a.out + ro)[i] = make_float4(o[0], o[1], o[2], o[3]);
+    if (a.out_h) {
+      half4 hv;
+#pragma unroll
+      for (int u = 0; u < 4; u++) hv[u] = (half_t)o[u];
+      reinterpret_cast<half4*>(a.out_h + ro)[i] = hv;
     }
   }
   if (a.lam_part) {
-    la = wave_sum_d(la);
-    lb = wave_sum_d(lb);
+    const double la = wave_sum_d(row_ok ? (double)pa : 0.0), lb = wave_sum_d(row_ok ? (double)pb : 0.0);
     if (lane == 0) { lsh[wave][0] = la; lsh[wave][1] = lb; }
   }
   __syncthreads();
   if (a.dgain_part)
-    for (int i = threadIdx.x; i < D; i += 256)
-      a.dgain_part[(size_t)blockIdx.x * D + i] = gsh[0][i] + gsh[1][i] + gsh[2][i] + gsh[3][i];
-  if (a.lam_part && threadIdx.x < 2)
-    a.lam_part[blockIdx.x * 2 + threadIdx.x] =
-        lsh[0][threadIdx.x] + lsh[1][threadIdx.x] + lsh[2][threadIdx.x] + lsh[3][threadIdx.x];
+    for (int i = threadIdx.x; i < D; i += 64 * kNormBwdRows) {
+      float g = gsh[0][i];
+#pragma unroll
+      for (int w = 1; w < kNormBwdRows; w++) g += gsh[w][i];
+      a.dgain_part[(size_t)blockIdx.x * D + i] = g;
+    }
+  if (a.lam_part && threadIdx.x < 2) {
+    double l = lsh[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kNormBwdRows; w++) l += lsh[w][threadIdx.x];
+    a.lam_part[blockIdx.x * 2 + threadIdx.x] = l;
+  }
 }
 
 // The gain form without the lambda, value-embedding and second-addend terms
@@ -247,6 +242,38 @@ __global__ __launch_bounds__(256) void reduce_dots_kernel(float* d0, float* d1, 
   }
 }
 
+// The lambda gradients of all layers: block l adds its layer's two norms'
+// partials (first the FFN norm's, part [2 l], then the attention norm's,
+// [2 l + 1], as the backward forms them) to dr[l] and dx[l].  One launch after
+// the layers instead of one behind each norm (26 of ~3.5 us per step).
+__global__ __launch_bounds__(256) void reduce_lams_kernel(float* dr, float* dx, const double* parts, int nblocks) {
+  __shared__ double sh[2][256];
+  const int l = blockIdx.x;
+  for (int i = 0; i < 2; i++) {
+    const double* part = parts + (size_t)(2 * l + i) * nblocks * 2;
+    double s0 = 0.0, s1 = 0.0;
+    for (int b = threadIdx.x; b < nblocks; b += 256) {
+      s0 += part[2 * b];
+      s1 += part[2 * b + 1];
+    }
+    sh[0][threadIdx.x] = s0;
+    sh[1][threadIdx.x] = s1;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+      if (threadIdx.x < o) {
+        sh[0][threadIdx.x] += sh[0][threadIdx.x + o];
+        sh[1][threadIdx.x] += sh[1][threadIdx.x + o];
+      }
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+      dr[l] += (float)sh[0][0];
+      dx[l] += (float)sh[1][0];
+    }
+    __syncthreads();
+  }
+}
+
 __global__ __launch_bounds__(256) void backout_bwd_kernel(float* ginj, double* part, const float* d, const float* xm,
                                                           const float* lam_p, size_t n) {
   __shared__ double sh[256];
@@ -317,7 +344,12 @@ __global__ __launch_bounds__(256) void embed_bwd_kernel(float* G, const float* d
   for (int i = lane; i < D; i += 64) atomicAdd(gr + i, xr[i]);
 }
 
-// one wave per token; lane = dim within a head, loop over heads
+// One wave per token; lane = dim within a head, loop over heads.  The gates
+// of all heads are formed at once, lane h head h's, and the gradients and
+// embeddings of kVeHeads heads are requested before the first is used (a
+// head at a time, each lane forming every gate: 17.9 us at 256 tokens x 12
+// heads; this: 9.9).
+constexpr int kVeHeads = 8;
 __global__ __launch_bounds__(256) void ve_bwd_kernel(float* gemb, float* ggate, float* ve_dx, const half_t* dv,
                                                      int ldv, const float* x, const float* emb, const float* vg,
                                                      const uint16_t* tok, int T, int D, int NH, int V) {
@@ -327,29 +359,51 @@ __global__ __launch_bounds__(256) void ve_bwd_kernel(float* gemb, float* ggate, 
   for (int i = lane; i < NH * 12; i += 64) gsh[wave][i] = 0.f;
   if (t < T) {
     const int tk = tok[t];
+    const bool hit = tk < V;
+    const float* er = emb + (size_t)(hit ? tk : 0) * D;
+    float* gr = gemb + (size_t)(hit ? tk : 0) * D;
     const float* xr = x + (size_t)t * D;
-    float xc[12];
+    const float* vgl = vg + (lane < NH ? lane : 0) * 12;
+    float xc[12], vgc[12];
 #pragma unroll
     for (int c = 0; c < 12; c++) xc[c] = xr[c];
-    float dxc[12];
 #pragma unroll
-    for (int c = 0; c < 12; c++) dxc[c] = 0.f;
-    for (int h = 0; h < NH; h++) {
-      float gp = 0.f;
+    for (int c = 0; c < 12; c++) vgc[c] = vgl[c];
+    float my_dgp = 0.f, my_act = 0.f;  // head `lane`'s
+    for (int h0 = 0; h0 < NH; h0 += kVeHeads) {
+      float dvd[kVeHeads], ev[kVeHeads];
 #pragma unroll
-      for (int c = 0; c < 12; c++) gp += vg[h * 12 + c] * xc[c];
-      const float act = (float)(1.0 / (1.0 + exp(-(double)gp)));
-      const float gate = 3.0f * act;
-      const float dvd = (float)dv[(size_t)t * ldv + h * 64 + lane];
-      const float ev = tk < V ? emb[(size_t)tk * D + h * 64 + lane] : 0.f;
-      if (tk < V) atomicAdd(gemb + (size_t)tk * D + h * 64 + lane, dvd * gate);
-      const float dg = wave_sum(dvd * ev);
-      const float dgp = dg * 3.0f * act * (1.f - act);
-      if (lane < 12) gsh[wave][h * 12 + lane] = dgp * xc[lane];
+      for (int u = 0; u < kVeHeads; u++) {
+        const int h = min(h0 + u, NH - 1);
+        dvd[u] = (float)dv[(size_t)t * ldv + h * 64 + lane];
+        ev[u] = hit ? er[h * 64 + lane] : 0.f;
+      }
+      if (h0 == 0) {
+        float gp = 0.f;
 #pragma unroll
-      for (int c = 0; c < 12; c++) dxc[c] += dgp * vg[h * 12 + c];
+        for (int c = 0; c < 12; c++) gp += vgc[c] * xc[c];
+        my_act = (float)(1.0 / (1.0 + exp(-(double)gp)));
+      }
+#pragma unroll
+      for (int u = 0; u < kVeHeads; u++) {
+        const int h = h0 + u;
+        if (h >= NH) break;
+        const float act = __shfl(my_act, h, 64);
+        if (hit) atomicAdd(gr + h * 64 + lane, dvd[u] * (3.0f * act));
+        const float dg = wave_sum_dpp(dvd[u] * ev[u]);
+        if (lane == h) my_dgp = dg * 3.0f * act * (1.f - act);
+      }
     }
-    if (lane < 12) ve_dx[(size_t)t * 12 + lane] = dxc[lane];
+    if (lane < NH) {
+#pragma unroll
+      for (int c = 0; c < 12; c++) gsh[wave][lane * 12 + c] = my_dgp * xc[c];
+    }
+    float dx = 0.f;  // channel `lane`'s, heads in order
+    for (int h = 0; h < NH; h++) {
+      const float d = __shfl(my_dgp, h, 64);
+      if (lane < 12) dx += d * vg[h * 12 + lane];
+    }
+    if (lane < 12) ve_dx[(size_t)t * 12 + lane] = dx;
   }
   __syncthreads();
   for (int i = threadIdx.x; i < NH * 12; i += 256)
@@ -610,13 +664,18 @@ hipError_t norm_bwd(const NormBwdArgs& a, hipStream_t s) {
                          !a.gx0 && !a.general && norm_bwd_fast();
   if (gain_only && a.addend) hipLaunchKernelGGL(norm_bwd_gain_kernel<true>, g, dim3(64 * kNormBwdRows), 0, s, a);
   else if (gain_only) hipLaunchKernelGGL(norm_bwd_gain_kernel<false>, g, dim3(64 * kNormBwdRows), 0, s, a);
-  else hipLaunchKernelGGL(norm_bwd_kernel, g, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(norm_bwd_kernel, g, dim3(64 * kNormBwdRows), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t reduce_partials_add(float* dst, const float* part, int nblocks, int n, hipStream_t s, bool overwrite) {
   hipLaunchKernelGGL(reduce_partials_kernel, dim3((n + 63) / 64), dim3(1024), 0, s, dst, part, nblocks, n,
                      overwrite ? 1 : 0);
+  return hipGetLastError();
+}
+
+hipError_t reduce_lams_add(float* dr, float* dx, const double* parts, int nblocks, int layers, hipStream_t s) {
+  hipLaunchKernelGGL(reduce_lams_kernel, dim3(layers), dim3(256), 0, s, dr, dx, parts, nblocks);
   return hipGetLastError();
 }
 
