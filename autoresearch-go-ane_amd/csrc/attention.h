@@ -28,6 +28,9 @@ struct AttnArgs {
 };
 
 hipError_t attention_fwd(const AttnArgs& a, hipStream_t stream);
+// The same for few (sequence, head) pairs (attention_few.hip); attention_fwd
+// calls it by its rule.  Does not stream pf.
+hipError_t attention_fwd_few(const AttnArgs& a, hipStream_t stream);
 
 // Backward of the fused attention (ane/train_full.go:261-316 for the
 // probabilities / ds recurrences, ane/common.go:229-270 for QK-norm).
@@ -53,5 +56,7 @@ struct AttnBwdArgs {
 
 // seq <= 256 (the whole sequence is staged in LDS twice).
 hipError_t attention_bwd(const AttnBwdArgs& a, hipStream_t stream);
+// The same for few (sequence, head) pairs, by attention_bwd's rule.
+hipError_t attention_bwd_few(const AttnBwdArgs& a, hipStream_t stream);
 
 }  // namespace ane

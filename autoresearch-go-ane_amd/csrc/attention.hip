@@ -533,6 +533,16 @@ void ane_k_attn_fwd15(AttnArgs a) {
 
 hipError_t attention_fwd(const AttnArgs& a, hipStream_t stream) {
   if (a.S <= 0 || a.S % 64 != 0 || a.S > 512 || a.NH <= 0 || a.nseq <= 0) return hipErrorInvalidValue;
+  if (a.hilo && a.S > 256) return hipErrorInvalidValue;
+  // Few heads: one 32-row q block per block, its keys split over four waves
+  // (attention_few.hip), while those blocks fit the GPU in one round; the
+  // kernels below walk up to S / 32 key blocks on one wave, longest at S > 256,
+  // where a second resident block per CU still pays.  us a launch (events),
+  // 12 layers' heads per sequence, below / few: S = 256 12 heads 14.3 / 10.9,
+  // 24 14.5 / 10.7, 36 14.5 / 15.0; S = 128 48 heads 11.6 / 9.0; S = 512 12
+  // heads 25.3 / 14.3, 24 24.8 / 20.4, 36 25.1 / 27.8; S = 320 48 heads 20.9 /
+  // 15.1, 72 20.4 / 22.7.
+  if ((long)a.nseq * a.NH * (a.S / 32) <= (a.S > 256 ? 512 : 256)) return attention_fwd_few(a, stream);
   const int npairs = a.S / 64;
   const int nw = npairs < 4 ? npairs : 4;  // q-block pairs per block
   dim3 grid((npairs + nw - 1) / nw, a.NH, a.nseq);
@@ -551,7 +561,6 @@ hipError_t attention_fwd(const AttnArgs& a, hipStream_t stream) {
     k.split_from = 256;
     grid = dim3(256 + 2 * (heads - 256), 1, 1);
   }
-  if (a.hilo && a.S > 256) return hipErrorInvalidValue;
   // ANE_ATT_15=0: the whole-head and half-head blocks above instead of 1.5 heads per block
   static const bool by15 = [] {
     const char* f = getenv("ANE_ATT_15");

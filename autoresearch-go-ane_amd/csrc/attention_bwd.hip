@@ -369,6 +369,13 @@ __global__ __launch_bounds__(PERQ ? 512 : 256) void attn_bwd_dkdv_kernel(AttnBwd
 
 hipError_t attention_bwd(const AttnBwdArgs& a, hipStream_t stream) {
   if (a.S <= 0 || a.S % 64 != 0 || a.S > 256 || a.NH <= 0 || a.nseq <= 0) return hipErrorInvalidValue;
+  if (a.hilo && !a.qkvt_lo) return hipErrorInvalidValue;
+  // Few heads: one 32-row block per block, both passes in one launch
+  // (attention_few.hip).  Forward and backward attention per layer, us, below
+  // / few backward: S = 256, 12 heads per sequence, 1 sequence 54 / 30, 4 58 /
+  // 52, 6 59 / 60; S = 64 16 sequences 33 / 31; split operands, S = 256, 1 104 /
+  // 66, 6 118 / 102, 8 127 / 121, 12 137 / 148.
+  if ((long)a.nseq * a.NH * (a.S / 32) <= (a.hilo ? 768 : 512)) return attention_bwd_few(a, stream);
   const int npairs = a.S / 64;
   const int nw = npairs < 4 ? npairs : 4;
   dim3 grid((npairs + nw - 1) / nw, a.NH, a.nseq);
@@ -378,7 +385,6 @@ hipError_t attention_bwd(const AttnBwdArgs& a, hipStream_t stream) {
     return !f || atoi(f) != 0;
   }();
   if (a.hilo) {
-    if (!a.qkvt_lo) return hipErrorInvalidValue;
     hipLaunchKernelGGL((attn_bwd_dq_kernel<256, true, false>), grid, dim3(64 * nw), 0, stream, a);
     hipLaunchKernelGGL((attn_bwd_dkdv_kernel<256, true, false>), grid, dim3(64 * nw), 0, stream, a);
   } else if (perq) {

@@ -1,0 +1,574 @@
+// Causal attention of few (sequence, head) pairs, forward and backward,
+// head_dim 64: the same functions as attention.hip and attention_bwd.hip,
+// for launches whose heads do not fill the GPU.
+//
+// Those kernels give a head one or two blocks, which stage its whole K and
+// V and walk up to 8 (16) key blocks one after the other: 12 heads keep 24 of
+// 256 CUs busy for the length of that chain (at 256 tokens 21-27 us a pass).
+// Here a block owns ONE 32-row block of a head, and its four waves take the
+// blocks on the other side in turn (key blocks kb = wave, wave + 4, ... of a
+// q block; q blocks of a key block in the dK/dV half), so the chain is a
+// quarter as long and heads x S/32 blocks share the work.  Nothing is staged for the
+// whole sequence: a wave reads its operand rows as MFMA fragments straight
+// from memory (row lane % 32, 16 bytes at dims 16 s + 8 (lane / 32)), applies
+// RoPE / QK-norm in those registers, and turns what is contracted over the
+// sequence (V; in the backward K, Q and dO) through a 32 x 64 LDS tile of
+// its own with ds_read_b64_tr_b16.  The waves meet once, at the end, in
+// wave order: the forward's running maxima and sums as in the online
+// softmax, the backward's gradients as plain sums.
+#include "attention.h"
+
+namespace ane {
+
+namespace {
+
+constexpr int HD = 64;
+constexpr int NWV = 4;         // waves that share a block's row block
+constexpr int TS = 72;         // LDS tile row stride (halves)
+constexpr float kLog2e = 1.4426950408889634f;
+
+struct Frag {  // one row's 32 of 64 values: dims 16 s + 8 g + [0, 8)
+  half8 v[4];
+};
+
+__device__ __forceinline__ Frag ld_frag(const half_t* row, int g) {
+  Frag f;
+#pragma unroll
+  for (int s = 0; s < 4; s++) f.v[s] = ld_h8(row + s * 16 + g * 8);
+  return f;
+}
+__device__ __forceinline__ void st_frag(half_t* row, const Frag& f, int g) {
+#pragma unroll
+  for (int s = 0; s < 4; s++) st_h8(row + s * 16 + g * 8, f.v[s]);
+}
+
+struct Angles {
+  float4 c[4], s[4];
+};
+__device__ __forceinline__ Angles ld_angles(const AttnArgs& a, int pos, int g) {
+  Angles r;
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    r.c[s] = *reinterpret_cast<const float4*>(a.rope_cos + pos * 32 + s * 8 + g * 4);
+    r.s[s] = *reinterpret_cast<const float4*>(a.rope_sin + pos * 32 + s * 8 + g * 4);
+  }
+  return r;
+}
+// RoPE, QK-norm (a row's two halves sit in lanes l and l ^ 32), fp16 and the fp16 residual
+template <bool HILO>
+__device__ __forceinline__ void turn(const AttnArgs& a, const Frag& raw, const Angles& an, Frag& hi, Frag& lo) {
+  float f[4][8];
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const float cs[4] = {an.c[s].x, an.c[s].y, an.c[s].z, an.c[s].w};
+    const float sn[4] = {an.s[s].x, an.s[s].y, an.s[s].z, an.s[s].w};
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+      const float e = (float)raw.v[s][2 * p], o = (float)raw.v[s][2 * p + 1];
+      f[s][2 * p] = e * cs[p] - o * sn[p];
+      f[s][2 * p + 1] = o * cs[p] + e * sn[p];
+    }
+  }
+  if (a.qknorm) {
+    float ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int p = 0; p < 8; p++) ss += f[s][p] * f[s][p];
+    ss += xor32_f(ss);
+    const float sc = 1.2f / sqrtf(ss * (1.0f / HD) + 1e-5f);
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int p = 0; p < 8; p++) f[s][p] *= sc;
+  }
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int p = 0; p < 8; p++) {
+      hi.v[s][p] = (half_t)f[s][p];
+      if constexpr (HILO) lo.v[s][p] = (half_t)(f[s][p] - (float)hi.v[s][p]);
+    }
+}
+
+// MFMA operand "32 dims x 16 positions" from a wave's [32 positions][64 dims]
+// tile: lane l receives dim d0 + l % 32 at positions 16 jh + 4 (l / 32) +
+// {0..3, 8..11}, the order in which a score accumulator's registers 8 jh ..
+// 8 jh + 7 hold its rows.
+__device__ __forceinline__ half8 tile_T(const half_t* tile, int d0, int jh, int lane) {
+  const int gg = lane >> 4, e = (lane >> 2) & 3, q = lane & 3;
+  const half_t* p = tile + (16 * jh + 4 * (gg >> 1) + e) * TS + d0 + 16 * (gg & 1) + 4 * q;
+  const short4v lohi[2] = {ds_read_tr16(p), ds_read_tr16(p + 8 * TS)};
+  return __builtin_bit_cast(half8, lohi);
+}
+// The wave's tile writes are in LDS order before its later reads; this keeps the compiler to it.
+__device__ __forceinline__ void tile_fence() { asm volatile("" ::: "memory"); }
+
+// HILO: scores from split operands (AttnArgs.hilo); LO: the fp16 residuals of q
+// and k are wanted (qkvt_lo).
+template <bool HILO, bool LO>
+__global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(HILO ? 1 : 2)))
+void attn_fwd_few_kernel(AttnArgs a) {
+  constexpr int OS = HD + 4;  // row stride of a partial output (floats)
+  __shared__ __attribute__((aligned(16))) char smem[NWV * 32 * OS * 4];
+  __shared__ float ml[NWV][2][32];
+  const int S = a.S, NH = a.NH, D = NH * HD, D3 = 3 * D;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 5, ql = lane & 31;
+  const int qb = gridDim.x - 1 - blockIdx.x, h = blockIdx.y;  // the longest first
+  const size_t tok0 = (size_t)blockIdx.z * S;
+  const half_t* base = a.qkv + tok0 * D3;
+  half_t* tile = reinterpret_cast<half_t*>(smem) + wave * (32 * TS);
+  const int q = qb * 32 + ql;
+
+  // requested together: q, and the wave's first key block (K, angles, V rows)
+  const Frag qraw = ld_frag(base + (size_t)q * D3 + h * HD, g);
+  const Angles qan = ld_angles(a, q, g);
+  const int vr = lane >> 3, vc = lane & 7;  // V: rows vr + 8 i, 16-byte chunk vc
+  Frag kraw;
+  Angles kan;
+  half8 vraw[4];
+  auto load = [&](int kb) {
+    kraw = ld_frag(base + (size_t)(kb * 32 + ql) * D3 + D + h * HD, g);
+    kan = ld_angles(a, kb * 32 + ql, g);
+#pragma unroll
+    for (int i = 0; i < 4; i++) vraw[i] = ld_h8(base + (size_t)(kb * 32 + vr + 8 * i) * D3 + 2 * D + h * HD + vc * 8);
+  };
+  if (wave <= qb) load(wave);
+  Frag qf, qlo;
+  turn<(HILO || LO)>(a, qraw, qan, qf, qlo);
+  if (wave == 0) {
+    if (a.qkvt) st_frag(a.qkvt + (tok0 + q) * D3 + h * HD, qf, g);
+    if (LO && a.qkvt_lo) st_frag(a.qkvt_lo + (tok0 + q) * 2 * D + h * HD, qlo, g);
+  }
+
+  const float sl2 = a.scale * kLog2e;
+  floatx16 o0, o1;
+#pragma unroll
+  for (int r = 0; r < 16; r++) o0[r] = o1[r] = 0.f;
+  float m = -INFINITY, lsum = 0.f;
+  for (int kb = wave; kb <= qb; kb += NWV) {
+    Frag kf, klo;
+    turn<(HILO || LO)>(a, kraw, kan, kf, klo);
+    half8 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = vraw[i];
+    if (a.ve_x) {
+      // value embeddings: v + 3 sigmoid(gate_h . x[:12]) * ve_embed[token]
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const size_t t = tok0 + kb * 32 + vr + 8 * i;
+        const float* xr = a.ve_x + t * D;
+        const int tk = a.tokens[t];
+        const bool hit = tk < a.vocab;
+        const float4* er = reinterpret_cast<const float4*>(a.ve_embed + (size_t)(hit ? tk : 0) * D + h * HD + vc * 8);
+        const float4 e0 = er[0], e1 = er[1];
+        float gp = 0.f;
+#pragma unroll
+        for (int c = 0; c < 12; c++) gp += a.ve_gate[h * 12 + c] * xr[c];
+        const float gate = hit ? 3.0f / (1.0f + __expf(-gp)) : 0.f;
+        const float ev[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[i][u] = hit ? (half_t)((float)v[i][u] + gate * ev[u]) : v[i][u];
+      }
+    }
+    if (kb == qb) {  // this block writes its own rows' training copies of k and v
+      if (a.qkvt) {
+        st_frag(a.qkvt + (tok0 + q) * D3 + D + h * HD, kf, g);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          st_h8(a.qkvt + (tok0 + kb * 32 + vr + 8 * i) * D3 + 2 * D + h * HD + vc * 8, v[i]);
+      }
+      if (LO && a.qkvt_lo) st_frag(a.qkvt_lo + (tok0 + q) * 2 * D + D + h * HD, klo, g);
+    }
+    tile_fence();
+#pragma unroll
+    for (int i = 0; i < 4; i++) st_h8(tile + (vr + 8 * i) * TS + vc * 8, v[i]);
+    tile_fence();
+    if (kb + NWV <= qb) load(kb + NWV);  // in flight during this block's products
+
+    floatx16 sacc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) sacc[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf.v[s], qf.v[s], sacc, 0, 0, 0);
+      if constexpr (HILO) {
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(klo.v[s], qf.v[s], sacc, 0, 0, 0);
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf.v[s], qlo.v[s], sacc, 0, 0, 0);
+      }
+    }
+    // sacc[r]: raw score of key kb*32 + 8*(r/4) + 4g + r%4, query q
+    if (kb == qb) {
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+        if ((8 * (r >> 2) + 4 * g + (r & 3)) > ql) sacc[r] = -INFINITY;
+    }
+    float mloc = sacc[0];
+#pragma unroll
+    for (int r = 1; r < 16; r++) mloc = fmaxf(mloc, sacc[r]);
+    mloc = fmaxf(mloc, xor32_f(mloc)) * sl2;  // scale > 0 keeps the order
+    const float mnew = fmaxf(m, mloc), alpha = __builtin_amdgcn_exp2f(m - mnew);
+    m = mnew;
+    lsum *= alpha;
+#pragma unroll
+    for (int r = 0; r < 16; r++) { o0[r] *= alpha; o1[r] *= alpha; }
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      sacc[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[r], sl2, -m));
+      lsum += sacc[r];
+    }
+#pragma unroll
+    for (int jh = 0; jh < 2; jh++) {
+      half8 pf;
+#pragma unroll
+      for (int u = 0; u < 8; u++) pf[u] = (half_t)sacc[8 * jh + u];
+      o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(tile_T(tile, 0, jh, lane), pf, o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(tile_T(tile, 32, jh, lane), pf, o1, 0, 0, 0);
+    }
+  }
+  lsum += xor32_f(lsum);
+  __syncthreads();  // the partial outputs take the tiles' place
+  float* om = reinterpret_cast<float*>(smem);
+  if (wave <= qb) {
+#pragma unroll
+    for (int rq = 0; rq < 4; rq++) {
+      float* d = om + (wave * 32 + ql) * OS + 8 * rq + 4 * g;
+      *reinterpret_cast<float4*>(d) = make_float4(o0[4 * rq], o0[4 * rq + 1], o0[4 * rq + 2], o0[4 * rq + 3]);
+      *reinterpret_cast<float4*>(d + 32) = make_float4(o1[4 * rq], o1[4 * rq + 1], o1[4 * rq + 2], o1[4 * rq + 3]);
+    }
+  }
+  if (g == 0) {
+    ml[wave][0][ql] = m;
+    ml[wave][1][ql] = lsum;
+  }
+  __syncthreads();
+  // thread: query tid / 8, dims 8 (tid % 8) .. + 7 (so a row leaves as 128 contiguous bytes)
+  const int oq = threadIdx.x >> 3, oc = threadIdx.x & 7;
+  float M = ml[0][0][oq];
+#pragma unroll
+  for (int w = 1; w < NWV; w++) M = fmaxf(M, ml[w][0][oq]);
+  float L = 0.f, o[8];
+#pragma unroll
+  for (int u = 0; u < 8; u++) o[u] = 0.f;
+#pragma unroll
+  for (int w = 0; w < NWV; w++) {
+    if (w > qb) break;  // uniform: that wave had no key block
+    const float sc = __builtin_amdgcn_exp2f(ml[w][0][oq] - M);
+    L += ml[w][1][oq] * sc;
+    const float* s = om + (w * 32 + oq) * OS + oc * 8;
+    const float4 x = *reinterpret_cast<const float4*>(s), y = *reinterpret_cast<const float4*>(s + 4);
+    o[0] += x.x * sc; o[1] += x.y * sc; o[2] += x.z * sc; o[3] += x.w * sc;
+    o[4] += y.x * sc; o[5] += y.y * sc; o[6] += y.z * sc; o[7] += y.w * sc;
+  }
+  const float inv = 1.0f / L;
+  half8 w8;
+#pragma unroll
+  for (int u = 0; u < 8; u++) w8[u] = (half_t)(o[u] * inv);
+  const size_t ot = tok0 + qb * 32 + oq;
+  st_h8(a.out + ot * D + h * HD + oc * 8, w8);
+  if (a.lse && oc == 0) a.lse[ot * NH + h] = (M + log2f(L)) / kLog2e;
+}
+
+
+// ---- backward ------------------------------------------------------------------
+// One launch for both passes (attention_bwd.hip has them as two): blocks
+// [0, S/32) of x are dQ's, one q block each, the rest dK/dV's, one key block
+// each.  delta = rowsum(dO * O) is formed by each wave for the rows it
+// reads, so neither half waits for the other.
+
+__device__ __forceinline__ float frag_dot(const Frag& a, const Frag& b) {
+  float d = 0.f;
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int p = 0; p < 8; p++) d += (float)a.v[s][p] * (float)b.v[s][p];
+  return d + xor32_f(d);
+}
+// a fragment's rows into a wave's [32][64] tile
+__device__ __forceinline__ void put_tile(half_t* tile, const Frag& f, int row, int g) {
+#pragma unroll
+  for (int s = 0; s < 4; s++) st_h8(tile + row * TS + s * 16 + g * 8, f.v[s]);
+}
+
+// Gradient of the transformed row (q or k) -> of the projection: the QK-norm
+// backward and the transposed rotation, as attention_bwd.hip's.  A lane holds
+// dims dt*32 + 8*(r/4) + 4g + r%4 of its row, lane l ^ 32 the others.
+__device__ __forceinline__ void few_post(float (&dv)[2][16], const half_t* raw, int pos, int g, const AttnBwdArgs& a) {
+  float cs[2][8], sn[2][8];
+  half4 hv[2][4];
+#pragma unroll
+  for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+    for (int rq = 0; rq < 4; rq++) {
+      const int d0 = dt * 32 + 8 * rq + 4 * g;
+      hv[dt][rq] = *reinterpret_cast<const half4*>(raw + d0);
+      const float2 c = *reinterpret_cast<const float2*>(a.rope_cos + pos * 32 + d0 / 2);
+      const float2 s = *reinterpret_cast<const float2*>(a.rope_sin + pos * 32 + d0 / 2);
+      cs[dt][2 * rq] = c.x; cs[dt][2 * rq + 1] = c.y;
+      sn[dt][2 * rq] = s.x; sn[dt][2 * rq + 1] = s.y;
+    }
+  if (a.qknorm) {
+    float pre[2][16], ss = 0.f, dot = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const float e = (float)hv[dt][i >> 1][2 * (i & 1)], o = (float)hv[dt][i >> 1][2 * (i & 1) + 1];
+        pre[dt][2 * i] = e * cs[dt][i] - o * sn[dt][i];
+        pre[dt][2 * i + 1] = o * cs[dt][i] + e * sn[dt][i];
+      }
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        ss += pre[dt][r] * pre[dt][r];
+        dot += dv[dt][r] * pre[dt][r];
+      }
+    ss += xor32_f(ss);
+    dot += xor32_f(dot);
+    const float rr = 1.0f / sqrtf(ss * (1.0f / HD) + 1e-5f);
+    const float coeff = dot * rr * rr * rr * (1.0f / HD) * a.qk_coef2;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) dv[dt][r] = dv[dt][r] * rr * 1.2f - coeff * pre[dt][r];
+  }
+  if (a.rope_bwd) {
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const float e = dv[dt][2 * i], o = dv[dt][2 * i + 1];
+        dv[dt][2 * i] = e * cs[dt][i] + o * sn[dt][i];
+        dv[dt][2 * i + 1] = o * cs[dt][i] - e * sn[dt][i];
+      }
+  }
+}
+
+__device__ __forceinline__ void few_store(half_t* dst, const float (&dv)[2][16], int g) {
+#pragma unroll
+  for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+    for (int rq = 0; rq < 4; rq++) {
+      half4 w;
+#pragma unroll
+      for (int u = 0; u < 4; u++) w[u] = (half_t)dv[dt][4 * rq + u];
+      *reinterpret_cast<half4*>(dst + dt * 32 + 8 * rq + 4 * g) = w;
+    }
+}
+
+// A wave's 64 x 32 accumulator pair into its partial slab, and the slabs of
+// all live waves summed in wave order (16 bytes per lane and access).
+__device__ __forceinline__ void put_part(float* slab, const floatx16& x, const floatx16& y, int lane) {
+  float4* d = reinterpret_cast<float4*>(slab);
+#pragma unroll
+  for (int rq = 0; rq < 4; rq++) {
+    d[rq * 64 + lane] = make_float4(x[4 * rq], x[4 * rq + 1], x[4 * rq + 2], x[4 * rq + 3]);
+    d[(4 + rq) * 64 + lane] = make_float4(y[4 * rq], y[4 * rq + 1], y[4 * rq + 2], y[4 * rq + 3]);
+  }
+}
+__device__ __forceinline__ void sum_parts(float (&o)[2][16], const float* slabs, int live, int lane) {
+#pragma unroll
+  for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
+  for (int w = 0; w < live; w++) {
+    const float4* s = reinterpret_cast<const float4*>(slabs + w * 2048);
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+      for (int rq = 0; rq < 4; rq++) {
+        const float4 v = s[(4 * dt + rq) * 64 + lane];
+        o[dt][4 * rq] += v.x; o[dt][4 * rq + 1] += v.y; o[dt][4 * rq + 2] += v.z; o[dt][4 * rq + 3] += v.w;
+      }
+  }
+}
+
+template <bool HILO>
+__global__ __launch_bounds__(64 * NWV) void attn_bwd_few_kernel(AttnBwdArgs a) {
+  // per wave: two tiles while it walks its blocks; after that, two partial slabs of 8 KB
+  __shared__ __attribute__((aligned(16))) char smem[NWV * 2 * 8192];
+  __shared__ __attribute__((aligned(16))) float rows[NWV][2][32];
+  const int S = a.S, NH = a.NH, D = NH * HD, D3 = 3 * D, nb = S / 32;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 5, ql = lane & 31;
+  const int h = blockIdx.y;
+  const size_t tok0 = (size_t)blockIdx.z * S;
+  const half_t* base = a.qkvt + tok0 * D3 + h * HD;
+  const half_t* lob = HILO ? a.qkvt_lo + tok0 * 2 * D + h * HD : nullptr;
+  half_t* tile0 = reinterpret_cast<half_t*>(smem) + wave * (2 * 32 * TS);
+  half_t* tile1 = tile0 + 32 * TS;
+  float* slabs = reinterpret_cast<float*>(smem);
+  const float sp = a.scale_p * kLog2e;
+
+  if ((int)blockIdx.x < nb) {  // ---- dQ: q block qb against key blocks wave, wave + 4, ... <= qb
+    const int qb = nb - 1 - blockIdx.x, q = qb * 32 + ql;
+    const size_t t = tok0 + q;
+    const Frag qf = ld_frag(base + (size_t)q * D3, g), df = ld_frag(a.dout + t * D + h * HD, g);
+    const Frag of = ld_frag(a.o + t * D + h * HD, g);
+    Frag qlo;
+    if constexpr (HILO) qlo = ld_frag(lob + (size_t)q * 2 * D, g);
+    const float lse2 = a.lse[t * NH + h] * kLog2e;
+    const float dd = frag_dot(df, of);
+    if (wave == 0 && g == 0) a.delta[t * NH + h] = dd;
+    floatx16 dq0, dq1;
+#pragma unroll
+    for (int r = 0; r < 16; r++) dq0[r] = dq1[r] = 0.f;
+    for (int kb = wave; kb <= qb; kb += NWV) {
+      const int key = kb * 32 + ql;
+      const Frag kf = ld_frag(base + (size_t)key * D3 + D, g), vf = ld_frag(base + (size_t)key * D3 + 2 * D, g);
+      Frag klo;
+      if constexpr (HILO) klo = ld_frag(lob + (size_t)key * 2 * D + D, g);
+      tile_fence();
+      put_tile(tile0, kf, ql, g);
+      tile_fence();
+      floatx16 sacc, dpacc;
+#pragma unroll
+      for (int r = 0; r < 16; r++) sacc[r] = dpacc[r] = 0.f;
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf.v[s], qf.v[s], sacc, 0, 0, 0);
+        if constexpr (HILO) {
+          sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(klo.v[s], qf.v[s], sacc, 0, 0, 0);
+          sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf.v[s], qlo.v[s], sacc, 0, 0, 0);
+        }
+        dpacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf.v[s], df.v[s], dpacc, 0, 0, 0);
+      }
+      float ds[16];
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const bool masked = kb == qb && (8 * (r >> 2) + 4 * g + (r & 3)) > ql;
+        const float p = masked ? 0.f : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[r], sp, -lse2));
+        ds[r] = p * (dpacc[r] - dd) * a.scale_ds;
+      }
+#pragma unroll
+      for (int jh = 0; jh < 2; jh++) {
+        half8 bf;
+#pragma unroll
+        for (int u = 0; u < 8; u++) bf[u] = (half_t)ds[8 * jh + u];
+        dq0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(tile_T(tile0, 0, jh, lane), bf, dq0, 0, 0, 0);
+        dq1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(tile_T(tile0, 32, jh, lane), bf, dq1, 0, 0, 0);
+      }
+    }
+    __syncthreads();  // the slabs take the tiles' place
+    if (wave <= qb) put_part(slabs + wave * 2048, dq0, dq1, lane);
+    __syncthreads();
+    if (wave != 0) return;
+    float dv[2][16];
+    sum_parts(dv, slabs, min(qb + 1, NWV), lane);
+    few_post(dv, a.qkv + t * D3 + h * HD, q, g, a);
+    few_store(a.dqkv + t * D3 + h * HD, dv, g);
+    return;
+  }
+
+  // ---- dK/dV: key block kb against q blocks kb + wave, kb + wave + 4, ... < nb
+  const int kb = blockIdx.x - nb, key = kb * 32 + ql;
+  const size_t t = tok0 + key;
+  const Frag kf = ld_frag(base + (size_t)key * D3 + D, g), vf = ld_frag(base + (size_t)key * D3 + 2 * D, g);
+  Frag klo;
+  if constexpr (HILO) klo = ld_frag(lob + (size_t)key * 2 * D + D, g);
+  floatx16 dk0, dk1, dv0, dv1;
+#pragma unroll
+  for (int r = 0; r < 16; r++) dk0[r] = dk1[r] = dv0[r] = dv1[r] = 0.f;
+  for (int qb = kb + wave; qb < nb; qb += NWV) {
+    const int q = qb * 32 + ql;
+    const Frag qf = ld_frag(base + (size_t)q * D3, g), df = ld_frag(a.dout + (tok0 + q) * D + h * HD, g);
+    const Frag of = ld_frag(a.o + (tok0 + q) * D + h * HD, g);
+    Frag qlo;
+    if constexpr (HILO) qlo = ld_frag(lob + (size_t)q * 2 * D, g);
+    const float ls = a.lse[(tok0 + q) * NH + h] * kLog2e, dl = frag_dot(df, of);
+    tile_fence();
+    put_tile(tile0, qf, ql, g);
+    put_tile(tile1, df, ql, g);
+    if (g == 0) {
+      rows[wave][0][ql] = ls;
+      rows[wave][1][ql] = dl;
+    }
+    tile_fence();
+    floatx16 sacc, dpacc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) sacc[r] = dpacc[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(qf.v[s], kf.v[s], sacc, 0, 0, 0);
+      if constexpr (HILO) {
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(qlo.v[s], kf.v[s], sacc, 0, 0, 0);
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(qf.v[s], klo.v[s], sacc, 0, 0, 0);
+      }
+      dpacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(df.v[s], vf.v[s], dpacc, 0, 0, 0);
+    }
+    // sacc[r] / dpacc[r]: query qb*32 + 8*(r/4) + 4g + r%4, key `key`
+    float pr[16], ds[16];
+#pragma unroll
+    for (int rq = 0; rq < 4; rq++) {
+      const float4 l4 = *reinterpret_cast<const float4*>(&rows[wave][0][8 * rq + 4 * g]);
+      const float4 d4 = *reinterpret_cast<const float4*>(&rows[wave][1][8 * rq + 4 * g]);
+      const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dlv[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int r = 4 * rq + u;
+        const bool masked = qb == kb && ql > (8 * rq + 4 * g + u);
+        const float p = masked ? 0.f : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[r], sp, -lv[u]));
+        pr[r] = p;
+        ds[r] = p * (dpacc[r] - dlv[u]) * a.scale_ds;
+      }
+    }
+#pragma unroll
+    for (int jh = 0; jh < 2; jh++) {
+      half8 pf, sf;
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        pf[u] = (half_t)pr[8 * jh + u];
+        sf[u] = (half_t)ds[8 * jh + u];
+      }
+      dv0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(tile_T(tile1, 0, jh, lane), pf, dv0, 0, 0, 0);
+      dv1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(tile_T(tile1, 32, jh, lane), pf, dv1, 0, 0, 0);
+      dk0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(tile_T(tile0, 0, jh, lane), sf, dk0, 0, 0, 0);
+      dk1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(tile_T(tile0, 32, jh, lane), sf, dk1, 0, 0, 0);
+    }
+  }
+  const int live = min(nb - kb, NWV);
+  __syncthreads();
+  if (wave < live) {
+    put_part(slabs + wave * 2048, dk0, dk1, lane);
+    put_part(slabs + (NWV + wave) * 2048, dv0, dv1, lane);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float dk[2][16];
+    sum_parts(dk, slabs, live, lane);
+    few_post(dk, a.qkv + t * D3 + D + h * HD, key, g, a);
+    few_store(a.dqkv + t * D3 + D + h * HD, dk, g);
+  } else if (wave == 1) {
+    float dv[2][16];
+    sum_parts(dv, slabs + NWV * 2048, live, lane);
+    few_store(a.dqkv + t * D3 + 2 * D + h * HD, dv, g);
+  }
+}
+
+}  // namespace
+
+hipError_t attention_fwd_few(const AttnArgs& a, hipStream_t stream) {
+  const dim3 grid(a.S / 32, a.NH, a.nseq);
+#define FEW(HILO_, LO_) hipLaunchKernelGGL((attn_fwd_few_kernel<HILO_, LO_>), grid, dim3(64 * NWV), 0, stream, a)
+  if (a.hilo) {
+    if (a.qkvt_lo) FEW(true, true);
+    else FEW(true, false);
+  } else if (a.qkvt_lo) {
+    FEW(false, true);
+  } else {
+    FEW(false, false);
+  }
+#undef FEW
+  return hipGetLastError();
+}
+
+hipError_t attention_bwd_few(const AttnBwdArgs& a, hipStream_t stream) {
+  const dim3 grid(2 * (a.S / 32), a.NH, a.nseq);
+  if (a.hilo) hipLaunchKernelGGL(attn_bwd_few_kernel<true>, grid, dim3(64 * NWV), 0, stream, a);
+  else hipLaunchKernelGGL(attn_bwd_few_kernel<false>, grid, dim3(64 * NWV), 0, stream, a);
+  return hipGetLastError();
+}
+
+}  // namespace ane
