@@ -110,9 +110,9 @@ class MoeLayer:
         """-> (out [T, D] fp32, expert ids int32 [T, 2], weights fp32 [T, 2])."""
         self._live()
         T, D = self.tokens, self.cfg.dim
-        out = np.zeros((T, D), np.float32)
-        idx = np.zeros((T, 2), np.int32)
-        w = np.zeros((T, 2), np.float32)
+        out = np.empty((T, D), np.float32)
+        idx = np.empty((T, 2), np.int32)
+        w = np.empty((T, 2), np.float32)
         self._check(self._lib.ane_moe_read_output(self._h, _f(out), idx.ctypes.data_as(C.POINTER(C.c_int32)),
                                                   _f(w)))
         return out, idx, w

@@ -27,6 +27,7 @@
 #include "../../include/ane_hip.h"
 #include "decode.h"
 #include "gemm.h"
+#include "host_copy.h"
 #include "rowops.h"
 
 using namespace ane;
@@ -69,6 +70,7 @@ struct ane_decoder {
   int D = 0, H = 0, NH = 0, NKV = 0, KVD = 0, N1 = 0, L = 0, V = 0, B = 0, C = 0;
   std::string err;
   hipStream_t stream = nullptr;
+  std::shared_ptr<HostPool> host_pool;  // from the first large copy on
   std::vector<void*> allocs;
   std::vector<DecLayerOff> off;
   int64_t off_embed = 0, off_gfinal = 0, nparams = 0;
@@ -481,9 +483,9 @@ int restore_start(ane_decoder* d, const char* op, int pos0) {
 int copy_out(ane_decoder* d, uint16_t* next_tok, float* logits) {
   const char* op = "copy out";
   if (next_tok) DCHK(op, hipMemcpyAsync(next_tok, d->tok_d, (size_t)d->nseq * 2, hipMemcpyDeviceToHost, d->stream));
-  if (logits)
-    DCHK(op, hipMemcpyAsync(logits, d->logits_d, (size_t)d->nseq * d->V * 4, hipMemcpyDeviceToHost, d->stream));
-  DCHK(op, hipStreamSynchronize(d->stream));
+  HostCopy hc(&d->host_pool, d->cfg.device, d->stream);
+  if (logits) DCHK(op, hc.down(logits, d->logits_d, (size_t)d->nseq * d->V * 4));
+  DCHK(op, hc.finish());
   return ANE_OK;
 }
 
@@ -532,7 +534,8 @@ extern "C" int ane_decode_set_params(ane_decoder* d, const float* params, int64_
   const int D = d->D, H = d->H, KVD = d->KVD, N1 = d->N1;
   const hipStream_t st = d->stream;
   DCHK(op, hipSetDevice(d->cfg.device));
-  DCHK(op, hipMemcpyAsync(d->P, params, (size_t)n * 4, hipMemcpyHostToDevice, st));
+  HostCopy hc(&d->host_pool, d->cfg.device, st);
+  DCHK(op, hc.up(d->P, params, (size_t)n * 4));
   for (int l = 0; l < d->L; l++) {
     const DecLayerOff& o = d->off[l];
     half_t* q = d->wqkv + (size_t)l * N1 * D;
@@ -551,7 +554,7 @@ extern "C" int ane_decode_set_params(ane_decoder* d, const float* params, int64_
     DCHK(op, weight_to_frag(d->fw2 + (size_t)l * D * H, d->w2 + (size_t)l * D * H, D, H, st));
   }
   DCHK(op, weight_to_frag(d->fembed, d->embed_h, d->V, D, st));
-  DCHK(op, hipStreamSynchronize(st));
+  DCHK(op, hc.finish());
   d->params_set = true;
   return ANE_OK;
 }

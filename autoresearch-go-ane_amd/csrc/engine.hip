@@ -225,6 +225,7 @@ static void free_all(ane_engine* e) {
   if (e->stream) (void)hipStreamSynchronize(e->stream);
   for (void* p : e->allocs) (void)hipFree(p);
   e->allocs.clear();
+  e->host_pool.reset();
   if (e->loss_host) (void)hipHostFree(e->loss_host);
   e->loss_host = nullptr;
   for (ProfEvent& pe : e->prof_events) {
@@ -621,10 +622,11 @@ extern "C" int ane_set_params(ane_engine* e, const float* params, int64_t n) {
   if (!params || n != e->pm.total)
     return eng_fail(e, ANE_ERR_ARG, "storiesane set params: len=%lld want=%lld", (long long)n,
                     (long long)e->pm.total);
-  HIPCHK("set params", hipMemcpyAsync(e->P, params, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
+  HostCopy hc(&e->host_pool, e->device, e->stream);
+  HIPCHK("set params", hc.up(e->P, params, (size_t)n * 4));
   int rc = refresh_shadows(e);
   if (rc) return rc;
-  HIPCHK("set params", hipStreamSynchronize(e->stream));
+  HIPCHK("set params", hc.finish());
   return ANE_OK;
 }
 
@@ -634,8 +636,9 @@ extern "C" int ane_get_params(ane_engine* e, float* params, int64_t n) {
   if (!params || n != e->pm.total)
     return eng_fail(e, ANE_ERR_ARG, "storiesane get params: len=%lld want=%lld", (long long)n,
                     (long long)e->pm.total);
-  HIPCHK("get params", hipMemcpyAsync(params, e->P, (size_t)n * 4, hipMemcpyDeviceToHost, e->stream));
-  HIPCHK("get params", hipStreamSynchronize(e->stream));
+  HostCopy hc(&e->host_pool, e->device, e->stream);
+  HIPCHK("get params", hc.down(params, e->P, (size_t)n * 4));
+  HIPCHK("get params", hc.finish());
   return ANE_OK;
 }
 
@@ -1027,8 +1030,9 @@ extern "C" int ane_eval_logits(ane_engine* e, const uint16_t* tokens, int64_t nt
   EpiParams p;
   p.C = e->logits; p.ldc = S; p.softcap = c.arch == ANE_ARCH_NANOCHAT; p.cap = 15.f;
   HIPCHK(op, eng_gemm(e, 4, e->embed_h, D, false, e->xh, D, false, V, S, D, EPI_LOGITS, p));
-  HIPCHK(op, hipMemcpyAsync(logits, e->logits, (size_t)V * S * 4, hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(op, stream_wait(e->stream));
+  HostCopy hc(&e->host_pool, e->device, e->stream);
+  HIPCHK(op, hc.down(logits, e->logits, (size_t)V * S * 4));
+  HIPCHK(op, hc.finish());
   return ANE_OK;
 }
 

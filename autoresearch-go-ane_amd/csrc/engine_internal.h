@@ -7,6 +7,7 @@
 
 #include "../../include/ane_hip.h"
 #include "gemm.h"
+#include "host_copy.h"
 #include "train_ops.h"
 
 struct LayerOff {
@@ -118,6 +119,7 @@ struct ane_engine {
   ane_model_cfg cfg{};
   ane_options opt{};
   int device = 0;
+  std::shared_ptr<ane::HostPool> host_pool;  // from the first large copy on
   bool dev_set = false;
   bool closed = false;
   std::string err;

@@ -1,0 +1,280 @@
+#include "host_copy.h"
+
+#include "hip_common.h"
+
+#include <string.h>
+
+#include <algorithm>
+
+namespace ane {
+
+namespace {
+inline void pause_cpu() { __builtin_ia32_pause(); }
+
+std::mutex g_pools_mu;
+constexpr int kMaxDevices = 64;
+constexpr uintptr_t kPage = (uintptr_t)2 << 20;  // a transparent huge page
+std::weak_ptr<HostPool> g_pools[kMaxDevices];
+}  // namespace
+
+std::shared_ptr<HostPool> host_pool(int device) {
+  if (device < 0 || device >= kMaxDevices) return nullptr;
+  std::lock_guard<std::mutex> lk(g_pools_mu);
+  if (auto p = g_pools[device].lock()) return p;
+  try {
+    std::shared_ptr<HostPool> p(new HostPool());
+    if (!p->init(device)) return nullptr;
+    g_pools[device] = p;
+    return p;
+  } catch (...) {
+    return nullptr;
+  }
+}
+
+bool HostPool::init(int device) {
+  // (a failure is cleared: the copy that asked goes through hipMemcpyAsync)
+  int prev = -1;
+  if (hipGetDevice(&prev) != hipSuccess || (prev != device && hipSetDevice(device) != hipSuccess)) {
+    (void)hipGetLastError();
+    return false;
+  }
+  struct Restore {
+    int prev, now;
+    ~Restore() {
+      if (prev != now) (void)hipSetDevice(prev);
+    }
+  } restore{prev, device};
+  if (hipHostMalloc((void**)&mem_, kSlots * kSlotBytes, hipHostMallocDefault) != hipSuccess) {
+    mem_ = nullptr;
+    (void)hipGetLastError();
+    return false;
+  }
+  for (int i = 0; i < kSlots; i++) {
+    slots_[i].mem = mem_ + i * kSlotBytes;
+    if (hipEventCreateWithFlags(&slots_[i].ev, hipEventDisableTiming) != hipSuccess) {
+      slots_[i].ev = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+  }
+  try {
+    const unsigned hw = std::thread::hardware_concurrency();
+    const int n = std::max(1, std::min(kThreads, hw > 2 ? (int)hw - 2 : 1));
+    for (int i = 0; i < n; i++) threads_.emplace_back([this] { run(); });
+  } catch (...) {
+    // fewer threads (or none): the copying thread works too
+  }
+  return true;
+}
+
+HostPool::~HostPool() {
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    stop_ = true;
+  }
+  cv_.notify_all();
+  for (std::thread& t : threads_) t.join();
+  for (Slot& s : slots_)
+    if (s.ev) {
+      if (s.in_flight) (void)hipEventSynchronize(s.ev);
+      (void)hipEventDestroy(s.ev);
+    }
+  if (mem_) (void)hipHostFree(mem_);
+}
+
+void HostPool::run() {
+  for (;;) {
+    {
+      std::unique_lock<std::mutex> lk(mu_);
+      cv_.wait(lk, [this] { return stop_ || awake_; });
+      if (stop_) return;
+    }
+    cv_.notify_one();  // the next sleeper (the caller wakes one thread, not all: ~12 us each)
+    while (awake_.load(std::memory_order_acquire) && !stop_)
+      if (!step())
+        for (int i = 0; i < 32; i++) pause_cpu();
+  }
+}
+
+bool HostPool::step() {
+  unsigned h = head_.load(std::memory_order_acquire);
+  while (h != tail_.load(std::memory_order_acquire)) {
+    const Task& t = ring_[h % kRing];  // what is read is this piece's if the claim succeeds: push() reuses no entry that head has not passed
+    void* dst = t.dst.load(std::memory_order_relaxed);
+    const void* src = t.src.load(std::memory_order_relaxed);
+    const size_t n = t.n.load(std::memory_order_relaxed);
+    std::atomic<int>* left = t.left.load(std::memory_order_relaxed);
+    if (head_.compare_exchange_weak(h, h + 1, std::memory_order_acq_rel)) {
+      if (src) {
+        memcpy(dst, src, n);
+      } else {  // first touch of a page about to be written
+        volatile char* c = (volatile char*)dst;
+        *c = *c;
+      }
+      left->fetch_sub(1, std::memory_order_release);
+      return true;
+    }
+  }
+  return false;
+}
+
+void HostPool::push(void* dst, const void* src, size_t n, std::atomic<int>* left) {
+  const unsigned t = tail_.load(std::memory_order_relaxed);
+  while (t - head_.load(std::memory_order_acquire) >= kRing) step();  // full: this thread works too
+  Task& k = ring_[t % kRing];
+  k.dst.store(dst, std::memory_order_relaxed);
+  k.src.store(src, std::memory_order_relaxed);
+  k.n.store(n, std::memory_order_relaxed);
+  k.left.store(left, std::memory_order_relaxed);
+  tail_.store(t + 1, std::memory_order_release);
+}
+
+void HostPool::wake() {
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    awake_ = true;
+  }
+  cv_.notify_one();
+}
+void HostPool::rest() { awake_.store(false, std::memory_order_release); }
+
+// ---- one call's copies ---------------------------------------------------------
+
+bool HostCopy::take(const void* host, size_t n) {
+  if (n < HostPool::kMinBytes || busy_) return false;
+  // memory the runtime already has pinned (or managed) is copied directly
+  hipPointerAttribute_t at;
+  memset(&at, 0, sizeof at);
+  if (hipPointerGetAttributes(&at, host) != hipSuccess) (void)hipGetLastError();
+  else if (at.type != hipMemoryTypeUnregistered) return false;
+  if (p_) return true;
+  if (!*handle_) *handle_ = host_pool(device_);
+  if (!*handle_ || !(*handle_)->use_.try_lock()) {
+    busy_ = true;
+    return false;
+  }
+  p_ = handle_->get();
+  p_->wake();
+  return true;
+}
+
+void HostCopy::drain(std::atomic<int>* left) {
+  while (left->load(std::memory_order_acquire) > 0)
+    if (!p_->step()) pause_cpu();
+}
+
+void HostCopy::split(char* dst, const char* src, size_t n, std::atomic<int>* left) {
+  const int k = (int)((n + HostPool::kTaskBytes - 1) / HostPool::kTaskBytes);
+  left->fetch_add(k, std::memory_order_relaxed);
+  for (size_t o = 0; o < n; o += HostPool::kTaskBytes)
+    p_->push(dst + o, src + o, std::min(HostPool::kTaskBytes, n - o), left);
+}
+
+hipError_t HostCopy::pass(HostPool::Slot* s) {
+  hipError_t h;
+  while ((h = hipEventQuery(s->ev)) == hipErrorNotReady)
+    if (!p_->step()) pause_cpu();
+  s->in_flight = false;
+  if (h == hipSuccess && s->host) split(s->host, s->mem, s->n, &s->left);
+  s->host = nullptr;
+  return h;
+}
+
+hipError_t HostCopy::pass_first() {
+  HostPool::Slot* s = &p_->slots_[pending_[first_]];
+  first_ = (first_ + 1) % HostPool::kSlots;
+  n_pending_--;
+  return pass(s);
+}
+
+hipError_t HostCopy::free_slot(HostPool::Slot** out) {
+  HostPool::Slot* s = &p_->slots_[p_->next_];
+  p_->next_ = (p_->next_ + 1) % HostPool::kSlots;
+  hipError_t h = hipSuccess;
+  if (s->in_flight) {  // the oldest: slots are used in turn
+    h = n_pending_ > 0 && &p_->slots_[pending_[first_]] == s ? pass_first() : pass(s);
+  }
+  drain(&s->left);
+  *out = s;
+  return h;
+}
+
+hipError_t HostCopy::up(void* dst, const void* src, size_t n) {
+  if (!take(src, n)) return hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st_);
+  for (size_t o = 0; o < n; o += HostPool::kSlotBytes) {
+    const size_t k = std::min(HostPool::kSlotBytes, n - o);
+    HostPool::Slot* s;
+    hipError_t h = free_slot(&s);
+    if (h != hipSuccess) return h;
+    split(s->mem, (const char*)src + o, k, &s->left);
+    drain(&s->left);
+    if ((h = hipMemcpyAsync((char*)dst + o, s->mem, k, hipMemcpyHostToDevice, st_)) != hipSuccess) return h;
+    if ((h = hipEventRecord(s->ev, st_)) != hipSuccess) return h;
+    s->in_flight = true;
+    s->host = nullptr;
+  }
+  return hipSuccess;
+}
+
+hipError_t HostCopy::down(void* dst, const void* src, size_t n) {
+  if (!take(dst, n)) return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st_);
+  // A buffer the caller has just allocated has no pages yet.  Each is touched
+  // by one thread before its bytes arrive: left to the copies, several
+  // threads would fault the same 2 MB page and each clear one for it.
+  const uintptr_t end = (uintptr_t)dst + n;
+  uintptr_t touch = n >= 2 * kPage ? (uintptr_t)dst : end;
+  auto touch_to = [&](uintptr_t upto) {
+    for (; touch < std::min(upto, end); touch = (touch | (kPage - 1)) + 1) {
+      p_->touched_.fetch_add(1, std::memory_order_relaxed);
+      p_->push((void*)touch, nullptr, 0, &p_->touched_);
+    }
+  };
+  for (size_t o = 0; o < n; o += HostPool::kSlotBytes) {
+    const size_t k = std::min(HostPool::kSlotBytes, n - o);
+    touch_to((uintptr_t)dst + o + 8 * kPage);
+    HostPool::Slot* s;
+    hipError_t h = free_slot(&s);
+    if (h != hipSuccess) return h;
+    if ((h = hipMemcpyAsync(s->mem, (const char*)src + o, k, hipMemcpyDeviceToHost, st_)) != hipSuccess) return h;
+    if ((h = hipEventRecord(s->ev, st_)) != hipSuccess) return h;
+    s->in_flight = true;
+    s->host = (char*)dst + o;
+    s->n = k;
+    pending_[(first_ + n_pending_++) % HostPool::kSlots] = (int)(s - p_->slots_);
+    // hand out what has arrived meanwhile
+    while (n_pending_ > 0 && hipEventQuery(p_->slots_[pending_[first_]].ev) == hipSuccess)
+      if ((h = pass_first()) != hipSuccess) return h;
+  }
+  return hipSuccess;
+}
+
+hipError_t HostCopy::finish() {
+  hipError_t h = hipSuccess;
+  if (p_) {
+    while (n_pending_ > 0) {
+      const hipError_t r = pass_first();
+      if (h == hipSuccess) h = r;
+    }
+    for (HostPool::Slot& s : p_->slots_) drain(&s.left);
+    drain(&p_->touched_);
+  }
+  const hipError_t r = stream_wait(st_);
+  return h == hipSuccess ? r : h;
+}
+
+HostCopy::~HostCopy() {
+  if (!p_) return;
+  // after an error: no destination is written once the call has returned
+  for (; n_pending_ > 0; n_pending_--, first_ = (first_ + 1) % HostPool::kSlots) {
+    HostPool::Slot& s = p_->slots_[pending_[first_]];
+    (void)hipEventSynchronize(s.ev);
+    s.in_flight = false;
+    s.host = nullptr;
+  }
+  for (HostPool::Slot& s : p_->slots_) drain(&s.left);
+  drain(&p_->touched_);
+  p_->rest();
+  p_->use_.unlock();
+}
+
+}  // namespace ane

@@ -29,6 +29,7 @@
 
 #include "../../include/ane_hip.h"
 #include "gemm.h"
+#include "host_copy.h"
 #include "rowops.h"
 
 using namespace ane;
@@ -271,6 +272,7 @@ struct ane_moe {
   int D = 0, H = 0, E = 0, TM = 0, RC = 0, T = 0;
   std::string err;
   hipStream_t stream = nullptr;
+  std::shared_ptr<HostPool> host_pool;  // from the first large copy on
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::vector<void*> allocs;
   bool params_set = false;
@@ -403,13 +405,14 @@ extern "C" int ane_moe_set_params(ane_moe* m, const float* params, int64_t n) {
   const size_t D = m->D, H = m->H;
   const hipStream_t st = m->stream;
   MCHK(op, hipSetDevice(m->cfg.device));
-  MCHK(op, hipMemcpyAsync(m->P, params, (size_t)n * 4, hipMemcpyHostToDevice, st));
+  HostCopy hc(&m->host_pool, m->cfg.device, st);
+  MCHK(op, hc.up(m->P, params, (size_t)n * 4));
   for (int e = 0; e < m->E; e++) {
     const float* base = m->P + (size_t)m->E * D + (size_t)e * 3 * H * D;
     MCHK(op, interleave_w13(m->w13 + (size_t)e * 2 * H * D, base, base + H * D, (int)H, (int)D, st));
     MCHK(op, f32_to_f16(m->w2 + (size_t)e * D * H, base + 2 * H * D, D * H, st));
   }
-  MCHK(op, hipStreamSynchronize(st));
+  MCHK(op, hc.finish());
   m->params_set = true;
   return ANE_OK;
 }
@@ -420,8 +423,9 @@ extern "C" int ane_moe_load_input(ane_moe* m, const float* x, int32_t tokens) {
   if (!x || tokens < 1 || tokens > m->TM)
     return mfail(m, ANE_ERR_ARG, "storiesane moe load input: tokens=%d want 1..%d", tokens, m->TM);
   MCHK(op, hipSetDevice(m->cfg.device));
-  MCHK(op, hipMemcpyAsync(m->x, x, (size_t)tokens * m->D * 4, hipMemcpyHostToDevice, m->stream));
-  MCHK(op, hipStreamSynchronize(m->stream));
+  HostCopy hc(&m->host_pool, m->cfg.device, m->stream);
+  MCHK(op, hc.up(m->x, x, (size_t)tokens * m->D * 4));
+  MCHK(op, hc.finish());
   m->T = tokens;
   return ANE_OK;
 }
@@ -478,10 +482,11 @@ extern "C" int ane_moe_read_output(ane_moe* m, float* out, int32_t* experts, flo
   if (!m || !m->stream) return ANE_ERR_STATE;
   if (m->T == 0) return mfail(m, ANE_ERR_STATE, "storiesane moe read output: no input loaded");
   MCHK(op, hipSetDevice(m->cfg.device));
-  if (out) MCHK(op, hipMemcpyAsync(out, m->out, (size_t)m->T * m->D * 4, hipMemcpyDeviceToHost, m->stream));
-  if (experts) MCHK(op, hipMemcpyAsync(experts, m->idx, (size_t)m->T * 8, hipMemcpyDeviceToHost, m->stream));
-  if (weights) MCHK(op, hipMemcpyAsync(weights, m->wts, (size_t)m->T * 8, hipMemcpyDeviceToHost, m->stream));
-  MCHK(op, hipStreamSynchronize(m->stream));
+  HostCopy hc(&m->host_pool, m->cfg.device, m->stream);
+  if (out) MCHK(op, hc.down(out, m->out, (size_t)m->T * m->D * 4));
+  if (experts) MCHK(op, hc.down(experts, m->idx, (size_t)m->T * 8));
+  if (weights) MCHK(op, hc.down(weights, m->wts, (size_t)m->T * 8));
+  MCHK(op, hc.finish());
   return ANE_OK;
 }
 

@@ -22,6 +22,7 @@
 #include "../../include/ane_objects.h"
 #include "attention.h"
 #include "gemm.h"
+#include "host_copy.h"
 #include "rowops.h"
 
 using namespace ane;
@@ -201,6 +202,8 @@ struct SeamBase {
   hipStream_t st = nullptr;
   std::vector<void*> allocs;
   bool closed = false;
+  std::shared_ptr<HostPool> pool;  // from the first large copy on
+  HostCopy* copies = nullptr;      // those of the call in hand (Copies)
 
   template <typename T>
   hipError_t alloc(T** p, size_t n) {
@@ -218,6 +221,7 @@ struct SeamBase {
     allocs.clear();
     if (st) (void)hipStreamDestroy(st);
     st = nullptr;
+    pool.reset();
     closed = true;
   }
   // the device and stream every call of the object uses
@@ -230,11 +234,21 @@ struct SeamBase {
     return hipSetDevice(device);
   }
   hipError_t up(void* dst, const void* src, size_t bytes) {
-    return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
+    return copies ? copies->up(dst, src, bytes) : hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
   }
   hipError_t down(void* dst, const void* src, size_t bytes) {
-    return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
+    return copies ? copies->down(dst, src, bytes) : hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
   }
+  // everything queued is done and every copy's destination written
+  hipError_t wait() { return copies ? copies->finish() : stream_wait(st); }
+};
+
+// The host copies of one call of an entered object.
+struct Copies {
+  SeamBase* b;
+  HostCopy hc;
+  explicit Copies(SeamBase* o) : b(o), hc(&o->pool, o->device, o->st) { b->copies = &hc; }
+  ~Copies() { b->copies = nullptr; }
 };
 
 int check_layer_shape(const char* op, int D, int H, int NH, int S, int max_seq) {
@@ -276,6 +290,7 @@ hipError_t alloc_shadows(SeamBase* b, LayerShadows* s, int D, int H) {
 
 hipError_t stage_layer(SeamBase* b, LayerShadows* s, const ane_layer_weights* w, int D, int H) {
   const size_t DD = (size_t)D * D;
+  Copies copies(b);
   hipError_t h;
   if ((h = stage_f16(b, s->wqkv, w->wq, DD, s->staging)) != hipSuccess) return h;
   if ((h = stage_f16(b, s->wqkv + DD, w->wk, DD, s->staging)) != hipSuccess) return h;
@@ -283,7 +298,7 @@ hipError_t stage_layer(SeamBase* b, LayerShadows* s, const ane_layer_weights* w,
   if ((h = stage_f16(b, s->wo, w->wo, DD, s->staging)) != hipSuccess) return h;
   if ((h = stage_f16(b, s->w1, w->w1, (size_t)H * D, s->staging)) != hipSuccess) return h;
   if ((h = stage_f16(b, s->w2, w->w2, (size_t)D * H, s->staging)) != hipSuccess) return h;
-  return stream_wait(b->st);  // the caller may free its host copies
+  return b->wait();  // the caller may free its host copies
 }
 
 // RoPE tables [S, 32] of the layer programs (theta 100000,
@@ -376,6 +391,7 @@ int layer_forward_call(ane_layer_fwd* f, float* out, const float* x, ane_layer_c
   const size_t DS = (size_t)D * S, HS = (size_t)H * S;
   hipStream_t st = f->st;
   SEAMCHK(op, f->enter());
+  Copies copies(f);
   SEAMCHK(op, f->up(f->xcf, x, DS * 4));
   SEAMCHK(op, layer_forward_device(f));
   SEAMCHK(op, (xpose<float, float>(f->cf, f->y, S, D, D, S, st)));
@@ -420,7 +436,7 @@ int layer_forward_call(ane_layer_fwd* f, float* out, const float* x, ane_layer_c
       SEAMCHK(op, tap(cache->gate, HS, f->cf2));
     }
   }
-  SEAMCHK(op, stream_wait(st));
+  SEAMCHK(op, f->wait());
   if (cache) {
     cache->att_taps_ready = 1;
     cache->ffn_taps_ready = 1;
@@ -584,6 +600,7 @@ extern "C" int ane_layer_backward_run_attention(ane_layer_bwd* lb, float* dx_nor
   const int D = lb->D, S = lb->S;
   const size_t DS = (size_t)D * S;
   hipStream_t st = lb->st;
+  Copies copies(lb);
   SEAMCHK(op, upload_cf(lb, lb->qkvt, 3 * D, q, D));
   SEAMCHK(op, upload_cf(lb, lb->qkvt + D, 3 * D, k, D));
   SEAMCHK(op, upload_cf(lb, lb->qkvt + 2 * D, 3 * D, v, D));
@@ -623,7 +640,7 @@ extern "C" int ane_layer_backward_run_attention(ane_layer_bwd* lb, float* dx_nor
   }
   SEAMCHK(op, (xpose<float, float>(lb->cf, lb->dxn, S, D, D, S, st)));
   SEAMCHK(op, lb->down(dx_norm, lb->cf, DS * 4));
-  SEAMCHK(op, stream_wait(st));
+  SEAMCHK(op, lb->wait());
   return ANE_OK;
 }
 
@@ -639,6 +656,7 @@ extern "C" int ane_layer_backward_run_ffn(ane_layer_bwd* lb, float* dx_norm, flo
   if (!dx_norm || !dh1 || !dffn || !h1) return seam_fail(ANE_ERR_ARG, "%s: null buffer", op);
   const int D = lb->D, H = lb->H, S = lb->S;
   hipStream_t st = lb->st;
+  Copies copies(lb);
   SEAMCHK(op, upload_cf(lb, lb->dffn, D, dffn, D));
   SEAMCHK(op, upload_cf(lb, lb->h1, H, h1, H));
   {
@@ -655,7 +673,7 @@ extern "C" int ane_layer_backward_run_ffn(ane_layer_bwd* lb, float* dx_norm, flo
   SEAMCHK(op, lb->down(dh1, lb->cf, (size_t)H * S * 4));
   SEAMCHK(op, (xpose<float, float>(lb->cf, lb->dxn, S, D, D, S, st)));
   SEAMCHK(op, lb->down(dx_norm, lb->cf, (size_t)D * S * 4));
-  SEAMCHK(op, stream_wait(st));
+  SEAMCHK(op, lb->wait());
   return ANE_OK;
 }
 
@@ -713,10 +731,11 @@ int offload_enter(const char* op, ane_offload* o, int piece) {
 
 hipError_t stage_embed(ane_offload* o, const float* embed) {
   const size_t n = (size_t)o->V * o->D;
+  Copies copies(o);
   hipError_t h = o->up(o->staging, embed, n * 4);
   if (h != hipSuccess) return h;
   if ((h = f32_to_f16(o->embed, o->staging, n, o->st)) != hipSuccess) return h;
-  return stream_wait(o->st);
+  return o->wait();
 }
 
 // logits [V, S] (device) = Embed x_norm, x_norm channel-first [D, S] from the host
@@ -808,12 +827,13 @@ extern "C" int ane_offload_run_rms_forward(ane_offload* o, float* out, const flo
   if (rc) return rc;
   if (!out || !x) return seam_fail(ANE_ERR_ARG, "%s: null buffer", op);
   const size_t DS = (size_t)o->D * o->S;
+  Copies copies(o);
   SEAMCHK(op, o->up(o->xcf, x, DS * 4));
   hipLaunchKernelGGL(cf_rms_fwd_kernel, dim3(o->S / 64), dim3(64 * kRmsRowLanes), 0, o->st, o->out, o->xcf, o->D,
                      o->S);
   SEAMCHK(op, hipGetLastError());
   SEAMCHK(op, o->down(out, o->out, DS * 4));
-  SEAMCHK(op, stream_wait(o->st));
+  SEAMCHK(op, o->wait());
   return ANE_OK;
 }
 
@@ -823,9 +843,10 @@ extern "C" int ane_offload_run_classifier_forward(ane_offload* o, float* logits,
   int rc = offload_enter(op, o, ANE_OFF_CLASSIFIER_FORWARD);
   if (rc) return rc;
   if (!logits || !x_norm) return seam_fail(ANE_ERR_ARG, "%s: null buffer", op);
+  Copies copies(o);
   SEAMCHK(op, classifier_device(o, x_norm));
   SEAMCHK(op, o->down(logits, o->logits, (size_t)o->V * o->S * 4));
-  SEAMCHK(op, stream_wait(o->st));
+  SEAMCHK(op, o->wait());
   return ANE_OK;
 }
 
@@ -836,10 +857,11 @@ extern "C" int ane_offload_run_classifier_softmax(ane_offload* o, float* probs, 
   if (rc) return rc;
   if (!(o->pieces & ANE_OFF_SOFTMAX)) return seam_fail(ANE_ERR_STATE, "%s: softmax kernel is unavailable", op);
   if (!probs || !x_norm) return seam_fail(ANE_ERR_ARG, "%s: null buffer", op);
+  Copies copies(o);
   SEAMCHK(op, classifier_device(o, x_norm));
   SEAMCHK(op, softmax_device(o));
   SEAMCHK(op, o->down(probs, o->logits, (size_t)o->V * o->S * 4));
-  SEAMCHK(op, stream_wait(o->st));
+  SEAMCHK(op, o->wait());
   return ANE_OK;
 }
 
@@ -850,10 +872,11 @@ extern "C" int ane_offload_run_softmax(ane_offload* o, float* probs) {
   if (rc) return rc;
   if (!probs) return seam_fail(ANE_ERR_ARG, "%s: null buffer", op);
   const size_t VS = (size_t)o->V * o->S;
+  Copies copies(o);
   SEAMCHK(op, o->up(o->logits, probs, VS * 4));
   SEAMCHK(op, softmax_device(o));
   SEAMCHK(op, o->down(probs, o->logits, VS * 4));
-  SEAMCHK(op, stream_wait(o->st));
+  SEAMCHK(op, o->wait());
   return ANE_OK;
 }
 
@@ -864,6 +887,7 @@ extern "C" int ane_offload_run_classifier_backward(ane_offload* o, float* dy, co
   if (rc) return rc;
   if (!dy || !dlogits) return seam_fail(ANE_ERR_ARG, "%s: null buffer", op);
   const size_t VS = (size_t)o->V * o->S;
+  Copies copies(o);
   SEAMCHK(op, o->up(o->staging, dlogits, VS * 4));
   SEAMCHK(op, f32_to_f16(o->dlh, o->staging, VS, o->st));
   // dy[d, t] = sum_v E[v, d] dlogits[v, t]: both operands read M-major,
@@ -877,7 +901,7 @@ extern "C" int ane_offload_run_classifier_backward(ane_offload* o, float* dy, co
   p.C = o->dycf; p.ldc = o->S;
   SEAMCHK(op, gemm_run(g, EPI_STORE_F, p, o->st, o->bwd_bm, o->bwd_bn));
   SEAMCHK(op, o->down(dy, o->dycf, (size_t)o->D * o->S * 4));
-  SEAMCHK(op, stream_wait(o->st));
+  SEAMCHK(op, o->wait());
   return ANE_OK;
 }
 
@@ -888,13 +912,14 @@ extern "C" int ane_offload_run_rms_backward(ane_offload* o, float* dx, const flo
   if (rc) return rc;
   if (!dx || !dy || !x) return seam_fail(ANE_ERR_ARG, "%s: null buffer", op);
   const size_t DS = (size_t)o->D * o->S;
+  Copies copies(o);
   SEAMCHK(op, o->up(o->xcf, x, DS * 4));
   SEAMCHK(op, o->up(o->dycf, dy, DS * 4));
   hipLaunchKernelGGL(cf_rms_bwd_kernel, dim3(o->S / 64), dim3(64 * kRmsRowLanes), 0, o->st, o->out, o->dycf,
                      o->xcf, o->D, o->S);
   SEAMCHK(op, hipGetLastError());
   SEAMCHK(op, o->down(dx, o->out, DS * 4));
-  SEAMCHK(op, stream_wait(o->st));
+  SEAMCHK(op, o->wait());
   return ANE_OK;
 }
 

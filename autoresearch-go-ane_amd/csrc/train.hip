@@ -844,8 +844,10 @@ extern "C" int ane_grads(ane_engine* e, const uint16_t* tokens, const uint16_t* 
   HIPCHK(op, fill_f32(e->tr.G, P, 0.f, e->stream));
   rc = backward_pass(e, nseq);
   if (rc) return rc;
-  HIPCHK(op, hipMemcpyAsync(grads, e->tr.G, P * 4, hipMemcpyDeviceToHost, e->stream));
+  HostCopy hc(&e->host_pool, e->device, e->stream);
+  HIPCHK(op, hc.down(grads, e->tr.G, P * 4));
   HIPCHK(op, fill_f32(e->tr.G, P, 0.f, e->stream));
+  HIPCHK(op, hc.finish());
   double mean = 0;
   rc = read_losses(e, nseq, nullptr, &mean);
   if (rc) return rc;
@@ -865,8 +867,9 @@ extern "C" int ane_set_grads(ane_engine* e, const float* grads, int64_t n, uint3
     return eng_fail(e, ANE_ERR_ARG, "storiesane set grads: len=%lld want=%lld", (long long)n, (long long)e->pm.total);
   int rc = ensure_train(e, op);
   if (rc) return rc;
-  HIPCHK(op, hipMemcpyAsync(e->tr.G, grads, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
-  HIPCHK(op, hipStreamSynchronize(e->stream));
+  HostCopy hc(&e->host_pool, e->device, e->stream);
+  HIPCHK(op, hc.up(e->tr.G, grads, (size_t)n * 4));
+  HIPCHK(op, hc.finish());
   e->state.pending_steps = pending;
   return ANE_OK;
 }
@@ -880,9 +883,10 @@ extern "C" int ane_get_opt_state(ane_engine* e, float* m, float* v, int64_t n) {
                     (long long)e->pm.total);
   int rc = ensure_train(e, op);
   if (rc) return rc;
-  if (m) HIPCHK(op, hipMemcpyAsync(m, e->tr.M, (size_t)n * 4, hipMemcpyDeviceToHost, e->stream));
-  if (v) HIPCHK(op, hipMemcpyAsync(v, e->tr.Vv, (size_t)n * 4, hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(op, hipStreamSynchronize(e->stream));
+  HostCopy hc(&e->host_pool, e->device, e->stream);
+  if (m) HIPCHK(op, hc.down(m, e->tr.M, (size_t)n * 4));
+  if (v) HIPCHK(op, hc.down(v, e->tr.Vv, (size_t)n * 4));
+  HIPCHK(op, hc.finish());
   return ANE_OK;
 }
 
@@ -895,11 +899,12 @@ extern "C" int ane_set_opt_state(ane_engine* e, const float* m, const float* v, 
                     (long long)e->pm.total);
   int rc = ensure_train(e, op);
   if (rc) return rc;
-  if (m) HIPCHK(op, hipMemcpyAsync(e->tr.M, m, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
+  HostCopy hc(&e->host_pool, e->device, e->stream);
+  if (m) HIPCHK(op, hc.up(e->tr.M, m, (size_t)n * 4));
   else HIPCHK(op, hipMemsetAsync(e->tr.M, 0, (size_t)n * 4, e->stream));
-  if (v) HIPCHK(op, hipMemcpyAsync(e->tr.Vv, v, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
+  if (v) HIPCHK(op, hc.up(e->tr.Vv, v, (size_t)n * 4));
   else HIPCHK(op, hipMemsetAsync(e->tr.Vv, 0, (size_t)n * 4, e->stream));
-  HIPCHK(op, hipStreamSynchronize(e->stream));
+  HIPCHK(op, hc.finish());
   return ANE_OK;
 }
 
@@ -916,8 +921,9 @@ extern "C" int ane_get_accum_grads(ane_engine* e, float* grads, int64_t n) {
     memset(grads, 0, (size_t)n * 4);
     return ANE_OK;
   }
-  HIPCHK(op, hipMemcpyAsync(grads, e->tr.G, (size_t)n * 4, hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(op, hipStreamSynchronize(e->stream));
+  HostCopy hc(&e->host_pool, e->device, e->stream);
+  HIPCHK(op, hc.down(grads, e->tr.G, (size_t)n * 4));
+  HIPCHK(op, hc.finish());
   return ANE_OK;
 }
 

@@ -1,0 +1,75 @@
+"""Copies between the caller's memory and the device through the pool of
+pinned slots: bit-exact round trips at sizes around a piece, a slot and the
+ring (layer weights set and read back, MoE activations), from several threads
+at once, and after every object that shared the pool is closed."""
+import ctypes as C
+import threading
+
+import numpy as np
+import pytest
+
+import ane
+from ane import _lib
+
+pytestmark = pytest.mark.gpu
+
+KB = 1024
+
+
+def engine(vocab, seed):
+    cfg = ane.Config(dim=64, hidden=64, heads=1, layers=1, vocab=vocab, seq=64, arch="llama2")
+    p = np.random.default_rng(seed).standard_normal(ane.param_count(cfg)).astype(np.float32)
+    return ane.Open(ane.Options(Config=cfg, Params=p)), p
+
+
+# 64 floats a vocabulary row (and 128 KiB of layer weights): below the pool's
+# least size, at it and past it, around one slot (4 MiB), past the ring of 8
+# slots, past twice that
+@pytest.mark.parametrize("vocab", [256, 512, 1024, 15808, 15872, 16384, 131072 + 6400, 65536 * 4 + 64])
+def test_params_round_trip(vocab):
+    eng, p = engine(vocab, vocab)
+    try:
+        for _ in range(2):
+            np.testing.assert_array_equal(eng.Params(), p)
+        q = np.ascontiguousarray(p[::-1])
+        eng.SetParams(q)
+        # an unaligned destination inside a larger buffer; what lies around it stays
+        buf = np.full(p.size + 5, np.float32(7))
+        rc = _lib.load().ane_get_params(eng._h, buf[3:].ctypes.data_as(C.POINTER(C.c_float)), p.size)
+        assert rc == 0
+        np.testing.assert_array_equal(buf[3:-2], q)
+        assert (buf[:3] == 7).all() and (buf[-2:] == 7).all()
+        m, v = (np.random.default_rng(s).random(p.size, dtype=np.float32) for s in (1, 2))
+        eng.SetOptState(m, v)
+        gm, gv = eng.OptState()
+        np.testing.assert_array_equal(gm, m)
+        np.testing.assert_array_equal(gv, v)
+    finally:
+        eng.Destroy()
+
+
+def test_threads_share_the_pool():
+    engs = [engine(40000 + 64 * i, i) for i in range(4)]
+    bad = []
+
+    def work(e, p):
+        try:
+            for _ in range(6):
+                if not np.array_equal(e.Params(), p):
+                    bad.append("params")
+                p = np.ascontiguousarray(np.roll(p, 1))
+                e.SetParams(p)
+        except Exception as x:  # reported below, in the test's own thread
+            bad.append(repr(x))
+
+    ts = [threading.Thread(target=work, args=ep) for ep in engs]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for e, _ in engs:
+        e.Destroy()
+    assert not bad
+    eng, p = engine(40000, 9)  # the pool again, after the last of them has gone
+    np.testing.assert_array_equal(eng.Params(), p)
+    eng.Destroy()
