@@ -551,13 +551,16 @@ hipError_t attention_fwd(const AttnArgs& a, hipStream_t stream) {
     const char* f = getenv("ANE_ATT_PERQ");
     return !f || atoi(f) != 0;
   }();
-  // One block of 4 pairs per head leaves 256 < heads < 512 unevenly spread
+  // One block of 4 pairs per head leaves 256 < heads <= 384 unevenly spread
   // over the 256 CUs (two blocks on some, one on the rest): the heads past
-  // 256 run as two half blocks, one beside each whole block.
+  // 256 run as two half blocks, one beside each whole block.  Past 384 the
+  // halves no longer fit beside them (two blocks per CU) and the whole
+  // blocks do, up to 512 (468 heads, halves / whole: 29.2 / 24.9 us, with
+  // value embeddings in half the layers 41.1 / 32.6).
   AttnArgs k = a;
   k.split_from = 0;
   const int heads = a.nseq * a.NH;
-  if (npairs == 4 && heads > 256 && heads < 512) {
+  if (npairs == 4 && heads > 256 && heads <= 384) {
     k.split_from = 256;
     grid = dim3(256 + 2 * (heads - 256), 1, 1);
   }
