@@ -152,7 +152,52 @@ __device__ __forceinline__ void wait_vm() {
 // has waited for the loads it needs; LDS reads/writes are drained here.
 __device__ __forceinline__ void barrier_keep_loads() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-__device__ __forceinline__ float softcap_f(float v, float cap) { return cap * tanhf(v / cap); }
+// cap * tanh(v / cap).  Every VALU instruction per logit costs the classifier
+// of 9984 tokens x 32000 ~10 us, so a lane's values of one column are capped
+// by the shortest form that holds for the largest of them (MA = max |v|, taken
+// over the wave): the Taylor series of tanh to x^7 below cap / 6, to x^13 below
+// 0.45 cap (both within 6e-8 of the value, half an ulp), else per value the
+// latter or 1 - 2 / (e^2x + 1) (within 2.6e-7; NaN and infinities pass through).
+// The cross-entropy GEMM at that size: tanhf 708 us, this 565, no softcap 484.
+struct Softcap {
+  float cap, inv, z1, c1, c2, c3, c4, c5, c6;  // series coefficients over powers of v^2
+  __device__ __forceinline__ explicit Softcap(float cap_) : cap(cap_), inv(1.f / cap_) {
+    z1 = inv * inv;
+    const float z2 = z1 * z1;
+    c1 = -1.f / 3.f * z1;
+    c2 = 2.f / 15.f * z2;
+    c3 = -17.f / 315.f * z2 * z1;
+    c4 = 62.f / 2835.f * z2 * z2;
+    c5 = -1382.f / 155925.f * z2 * z2 * z1;
+    c6 = 21844.f / 6081075.f * z2 * z2 * z2;
+  }
+  __device__ __forceinline__ float low(float v) const {
+    const float z = v * v;
+    return __builtin_fmaf(v * z, __builtin_fmaf(__builtin_fmaf(c3, z, c2), z, c1), v);
+  }
+  __device__ __forceinline__ float mid(float v) const {
+    const float z = v * v;
+    float p = __builtin_fmaf(c6, z, c5);
+    p = __builtin_fmaf(p, z, c4);
+    p = __builtin_fmaf(p, z, c3);
+    p = __builtin_fmaf(p, z, c2);
+    p = __builtin_fmaf(p, z, c1);
+    return __builtin_fmaf(v * z, p, v);
+  }
+  __device__ __forceinline__ float any(float v) const {
+    const float av = fabsf(v);
+    const float e = __builtin_amdgcn_exp2f(av * (2.8853900817779268f * inv));  // 2 log2(e) |v| / cap
+    const float big = copysignf(cap * __builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(e + 1.f), 1.f), v);
+    return av < 0.45f * cap ? mid(v) : big;
+  }
+  // f(value) over a lane's values of one column; ma = max |value| of the lane
+  template <typename F>
+  __device__ __forceinline__ void over(float ma, F f) const {
+    if (__all(ma < cap * (1.f / 6.f))) f([this](float v) { return low(v); });
+    else if (__all(ma < 0.45f * cap)) f([this](float v) { return mid(v); });
+    else f([this](float v) { return any(v); });
+  }
+};
 
 // logistic function with the hardware reciprocal (1 ulp) instead of an IEEE
 // division sequence; its results feed fp16 stores or fp32 gates
@@ -262,16 +307,27 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[TM][TN], const GemmArgs
         }
   } else if constexpr (EPI == EPI_LOGITS) {
     float* C = (float*)e.C;
+    if (e.softcap) {
+      const Softcap sc(e.cap);
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          float ma = 0.f;
+#pragma unroll
+          for (int r = 0; r < 16; r++) ma = fmaxf(ma, fabsf(acc[i][j][r]));
+          sc.over(ma, [&](auto f) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r]);
+          });
+        }
+    }
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
       for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          float v = acc[i][j][r];
-          if (e.softcap) v = softcap_f(v, e.cap);
-          C[(size_t)ROW(i, r) * e.ldc + COL(j)] = v;
-        }
+        for (int r = 0; r < 16; r++) C[(size_t)ROW(i, r) * e.ldc + COL(j)] = acc[i][j][r];
   } else if constexpr (EPI == EPI_RESID) {
     float* C = (float*)e.C;
     float* C2 = (float*)e.C2;
@@ -468,28 +524,47 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[TM][TN], const GemmArgs
       // compare against a constant per register
       const int tsel = (tg_pre ? tg_pre[j] : (int)e.targets[n]) - ROW(0, 0);
       const bool hit = tsel >= 0 && tsel < 32 * TM && (tsel & 4) == 0;
-      const float rr_col = EPI == EPI_CE_RR ? rr_s[nl] : 1.f;
+      // 1 / rms of the column is folded into the exponentials' factor, the
+      // maximum and the target (a multiplication less per logit)
+      float scale = EPI == EPI_CE_RR ? rr_s[nl] : 1.f;
       float mx = -INFINITY, tv = 0.f;
+      if (e.softcap) {
+        float ma = 0.f;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            if constexpr (EPI == EPI_CE_RR) acc[i][j][r] *= scale;
+            ma = fmaxf(ma, fabsf(acc[i][j][r]));
+          }
+        scale = 1.f;
+        Softcap(e.cap).over(ma, [&](auto f) {
+#pragma unroll
+          for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r]);
+        });
+      }
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          float v = acc[i][j][r];
-          if constexpr (EPI == EPI_CE_RR) v *= rr_col;
-          if (e.softcap) v = softcap_f(v, e.cap);
-          acc[i][j][r] = v;
-          mx = fmaxf(mx, v);
-          tv = (32 * i + 8 * (r >> 2) + (r & 3)) == tsel ? v : tv;
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        for (int r = 0; r < 16; r++) mx = fmaxf(mx, acc[i][j][r]);
+      if (__any(hit)) {  // few waves hold a target of these 32 columns (12% at vocabulary 32000)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) tv = (32 * i + 8 * (r >> 2) + (r & 3)) == tsel ? acc[i][j][r] : tv;
+        tv *= scale;
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * scale;
       // sum exp(v - max) as exp2(v log2e - max log2e): one FMA per value
       constexpr float kLog2e = 1.4426950408889634f;
-      const float mxl = mx * kLog2e;
+      const float mxl = mx * kLog2e, fac = scale * kLog2e;
       float s = 0.f;
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) s += __builtin_amdgcn_exp2f(__builtin_fmaf(acc[i][j][r], kLog2e, -mxl));
+        for (int r = 0; r < 16; r++) s += __builtin_amdgcn_exp2f(__builtin_fmaf(acc[i][j][r], fac, -mxl));
       s += __shfl_xor(s, 32, 64);
       if (hit) e.tgt_logit[n] = tv;  // exactly one lane of the grid holds (tg, n)
       if (lane < 32) red[wm * BN + nl] = make_float2(mx, s);
@@ -522,17 +597,31 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[TM][TN], const GemmArgs
       // per register one compare against a constant each
       const int tsel = e.targets[n] - ROW(0, 0), vend = e.vocab - ROW(0, 0);
       const float lsel = e.lse[n] * kLog2e, cs = e.colscale[n];
+      if (e.softcap) {
+        float ma = 0.f;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) ma = fmaxf(ma, fabsf(acc[i][j][r]));
+        Softcap(e.cap).over(ma, [&](auto f) {
+#pragma unroll
+          for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r]);
+        });
+      }
+      const float icap = 1.f / e.cap;
 #pragma unroll
       for (int i = 0; i < TM; i++) {
         half_t hv[16];
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const int mo = 32 * i + 8 * (r >> 2) + (r & 3);
-          float v = acc[i][j][r], dsc = 1.f;
+          const float v = acc[i][j][r];
+          float dsc = 1.f;
           if (e.softcap) {
-            float th = tanhf(v / e.cap);
-            v = e.cap * th;
-            dsc = 1.f - th * th;
+            const float th = v * icap;
+            dsc = __builtin_fmaf(-th, th, 1.f);
           }
           float d = __builtin_amdgcn_exp2f(__builtin_fmaf(v, kLog2e, -lsel)) - (mo == tsel ? 1.f : 0.f);
           d = mo < vend ? d * cs * dsc : 0.f;
