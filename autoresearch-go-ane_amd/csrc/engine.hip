@@ -900,10 +900,10 @@ int head_loss(ane_engine* e, int nseq, float* colscale, float dscale) {
   EpiParams p;
   p.targets = e->tgt; p.partial = e->partial; p.tgt_logit = e->tgt_logit;
   p.softcap = c.arch == ANE_ARCH_NANOCHAT; p.cap = 15.f; p.vocab = V;
-  // block rows: 256 (8-wave 256x256 tiles) once that still gives >= 512
-  // blocks, else the open-time size; the partial buffer holds V / ce_bm rows
+  // block rows: 256 (8-wave 256x256 tiles) once they nearly fill the CUs
+  // (gemm_ce_big), else the open-time size; the partial buffer holds V / ce_bm rows
   int bm = e->ce_bm, bn = 0;
-  if (V % 256 == 0 && T % 256 == 0 && (long)(V / 256) * (T / 256) >= 512) bm = bn = 256;
+  if (gemm_ce_big(V, T)) bm = bn = 256;
   const int np = V / bm;
   if (e->fwd_rr_nparts > 0) {  // the final norm deferred into the classifier
     p.rr_part = e->ssq_part; p.rr_ld = T; p.rr_nparts = e->fwd_rr_nparts; p.rr_dim = D;

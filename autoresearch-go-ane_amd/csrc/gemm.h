@@ -142,6 +142,14 @@ int gemm_pick_thin_splits(int M, int N, int K, size_t ws_cap);
 bool gemm_thin_aligned(const GemmArgs& g, int epi, const EpiParams& e);
 hipError_t gemm_thin_run(const ThinTile& t, const GemmArgs& g, int epi, const EpiParams& e, hipStream_t stream);
 
+// Whether the classifier of T tokens takes 256x256 tiles: from 240 blocks, nearly
+// the CUs (vocabulary 32000, us, before / 256x256: 512 tokens, 250 blocks, 35.8 /
+// 25.8; 768, 375 blocks, 50.9 / 46.1; 1024 68.5 / 49.5; below, 256 tokens on 125
+// blocks, 128x128 tiles are better: 17.2 against 21.2).
+inline bool gemm_ce_big(int V, int T) {
+  return V % 256 == 0 && T % 256 == 0 && (long)(V / 256) * (T / 256) >= 240;
+}
+
 // Tile the heuristic picks; nonzero *bm / *bn on entry are kept as
 // constraints (set both to 0 for a free choice).  0 = no tile fits.
 void gemm_pick_tile(int M, int N, int K, int epi, int* bm, int* bn);

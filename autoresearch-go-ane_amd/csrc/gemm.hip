@@ -27,10 +27,15 @@ void gemm_pick_tile(int M, int N, int K, int epi, int* pbm, int* pbn) {
   // 925 vs 817 TFLOP/s for 128x128, at M = 4096: 953 vs 809; classifier 885
   // vs 801), 128x128 from 512 blocks (the SwiGLU-backward GEMM at M = 4096:
   // 18.0 vs 21.4 us for 128x64), 128x64 at N = 768 with K <= 2048, 64x64
-  // for narrow outputs with long K.  A nonzero
+  // for narrow outputs with long K.  128x128 is taken from 385 blocks: there
+  // the 128x64 and 64x128 tiles pass the 768 blocks that are resident at
+  // three per CU and begin a second round (us, 128x64 / 128x128: 9216 x 768 x
+  // 768 26.6 / 21.8, 9216 x 768 x 2048 53.6 / 38.9, 3328 x 2048 x 768 24.0 /
+  // 18.7, 1664 x 4096 x 768 SwiGLU (64x128) 21.9 / 15.9); at 384 (8192 x 768)
+  // they fit exactly.  A nonzero
   // *pbm / *pbn on entry is a constraint the chosen tile keeps (callers
   // size buffers by it).
-  static const int cand[][3] = {{256, 256, 256}, {128, 128, 512}, {128, 64, 600}, {64, 128, 600},
+  static const int cand[][3] = {{256, 256, 256}, {128, 128, 385}, {128, 64, 600}, {64, 128, 600},
                                 {256, 128, 600},  {128, 256, 600},  {256, 64, 600}, {64, 64, 0}};
   constexpr int NCAND = 8;
   const int want_bm = *pbm, want_bn = *pbn;
@@ -44,6 +49,11 @@ void gemm_pick_tile(int M, int N, int K, int epi, int* pbm, int* pbn) {
       (!want_bn || want_bn == 192)) {
     *pbm = 128;
     *pbn = 192;
+    return;
+  }
+  if ((epi == EPI_CE || epi == EPI_DLOGITS || epi == EPI_LOGITS) && gemm_ce_big(M, N) &&
+      (!want_bm || want_bm == 256) && (!want_bn || want_bn == 256)) {
+    *pbm = *pbn = 256;
     return;
   }
   int fbm = 0, fbn = 0;
