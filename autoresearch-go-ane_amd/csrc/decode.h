@@ -18,7 +18,7 @@ namespace ane {
 constexpr int kDecRows = 64;    // token rows of a decode step (max sequences)
 constexpr int kDecChunk = 256;  // keys per decode-attention split
 constexpr int kDecWideChunk = 1152;   // keys per split of the 1024-thread form (9 passes of 128)
-constexpr int kDecWideMinBlocks = 192;  // batch x kv heads from which that form is chosen
+constexpr int kDecWideMinBlocks = 192;  // batch x kv heads from which that form is chosen as a launch of its own
 
 // MFMA-fragment-major layout of the decode-step operands.  A 32x32x16 MFMA
 // operand lane l takes row l%32 and eight k-values; with the k-slot map
@@ -169,6 +169,7 @@ struct TailArgs {
   int* err;                 // set when a wait times out; later launches exit at once
   unsigned spin_limit;      // polls before a wait times out (kDecTailSpin; 0: every wait fails)
   int D, H, N1, layer, L;
+  int nb;                   // sequences (1..64): rows from nb on hold nothing that is used
   int b_wo, b_13, b_w2, b_q;  // blocks per phase: D/32, H/32, D/32, N1/32 (0 on the last layer)
   // data-polling form (poll != 0): the two buffer sets (tail_set_bytes each,
   // every dword kTailStale at open); xg_ffn, ssq_wo, ssq_w2 and sync above
@@ -187,7 +188,10 @@ struct TailArgs {
   DecAttnArgs att_next;
 };
 // Whether the attention of `a` can run inside the chain's launch (the wide
-// form with one split, G <= kGMax).
+// form with one split, G <= kGMax, whatever the batch: its K / V loads are
+// under way while the chain runs, and two launches per layer are saved.  A step
+// with the split form beside the chain against this, 3 sequences at 192..256:
+// 385, 356 us; 47 at 1024..1088: 530, 409).
 bool dec_attention_fusable(const DecAttnArgs& a);
 constexpr int kDecTailSync = 64;
 constexpr unsigned kDecTailSpin = 1u << 20;  // polls of ~100 cycles: ~50 ms

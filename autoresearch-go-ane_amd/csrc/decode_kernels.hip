@@ -859,7 +859,7 @@ hipError_t dec_norm(const float* x, half_t* xn, const float* g, int nb, int D, h
 bool dec_attention_fusable(const DecAttnArgs& a) {
   if (a.NKV <= 0 || a.NH % a.NKV || a.NH / a.NKV > kGMax) return false;
   const int wsplit = (a.max_ctx + kDecWideChunk - 1) / kDecWideChunk;
-  return wsplit == 1 && wsplit <= a.nsplit && (a.form == 1 || (a.form == 0 && a.nb * a.NKV >= kDecWideMinBlocks));
+  return wsplit == 1 && wsplit <= a.nsplit && a.form != 2;
 }
 
 hipError_t dec_attention(const DecAttnArgs& a, hipStream_t s) {

@@ -119,10 +119,12 @@ __device__ __forceinline__ Span wave_span(int nwin, int nwave, int wave) {
   return Span{a, min(b - a, MAXW)};
 }
 
-// One wave's 64 x 32 partial over its windows: weights of column group cg
+// One wave's 32 RT x 32 partial over its windows: weights of column group cg
 // (fragment-major, nwin windows per group) preloaded by load_w, activations
-// X (activation fragments) loaded after the dependency wait by mma.
-template <int MAXW>
+// X (activation fragments) loaded after the dependency wait by mma.  Rows
+// from nb on hold no sequence: their lanes repeat row nb - 1 (the same cache
+// lines), and their results go nowhere.
+template <int MAXW, int RT>
 struct WaveGemm {
   half8 w[4 * MAXW];
   floatx16 c0, c1;
@@ -135,75 +137,89 @@ struct WaveGemm {
     }
   }
   // coherent: X was written inside this launch (device-coherent loads)
-  __device__ __forceinline__ void mma(const half_t* X, Span sp, bool coherent) {
-    const int lane8 = threadIdx.x % 64 * 8;
+  __device__ __forceinline__ void mma(const half_t* X, Span sp, bool coherent, int nb) {
+    const int lane0 = frag_lane(nb, 0), lane1 = RT == 2 ? frag_lane(nb, 1) : lane0;
     half8 p[4 * MAXW], q[4 * MAXW];
 #pragma unroll
     for (int s = 0; s < 4 * MAXW; s++) {
       const int f = (sp.w0 + min(s >> 2, max(sp.nw - 1, 0))) * 4 + (s & 3);
       if (coherent) {
-        p[s] = ld_ch8(X, (uint32_t)(f * 1024 + lane8));
-        q[s] = ld_ch8(X, (uint32_t)(f * 1024 + 512 + lane8));
+        p[s] = ld_ch8(X, (uint32_t)(f * 1024 + lane0));
+        if (RT > 1) q[s] = ld_ch8(X, (uint32_t)(f * 1024 + 512 + lane1));
       } else {
-        p[s] = ld_h8(X + (size_t)f * 1024 + lane8);
-        q[s] = ld_h8(X + (size_t)f * 1024 + 512 + lane8);
+        p[s] = ld_h8(X + (size_t)f * 1024 + lane0);
+        if (RT > 1) q[s] = ld_h8(X + (size_t)f * 1024 + 512 + lane1);
       }
     }
-#pragma unroll
-    for (int r = 0; r < 16; r++) { c0[r] = 0.f; c1[r] = 0.f; }
-#pragma unroll
-    for (int s = 0; s < 4 * MAXW; s++) {
-      if ((s >> 2) < sp.nw) {  // wave-uniform: surplus windows contribute nothing
-        c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(p[s], w[s], c0, 0, 0, 0);
-        c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(q[s], w[s], c1, 0, 0, 0);
-      }
-    }
+    compute(sp, p, q);
   }
   // Data-polling form: the activation fragments into px / qx (device-coherent
   // loads); true when no dword of this lane's is stale.  compute() then
   // runs the MFMAs on them.
   half8 px[4 * MAXW], qx[4 * MAXW];
-  __device__ __forceinline__ bool load_x(const half_t* X, Span sp) {
+  // this lane's offset in a fragment of row tile t: row lane % 32, at most nb - 1
+  static __device__ __forceinline__ int frag_lane(int nb, int t) {
+    const int l = threadIdx.x & 63;
+    return (min(l & 31, max(nb - 1 - 32 * t, 0)) + (l & 32)) * 8;
+  }
+  __device__ __forceinline__ bool load_x(const half_t* X, Span sp, int nb) {
     // recomputed each round (opaque to loop-invariant hoisting): the load
     // offsets then hold no register while the round's data is in flight
-    int lane8 = threadIdx.x % 64 * 8;
-    asm volatile("" : "+v"(lane8));
+    int lane0 = frag_lane(nb, 0);
+    asm volatile("" : "+v"(lane0));
+    int lane1 = lane0;
+    if constexpr (RT == 2) {
+      lane1 = frag_lane(nb, 1);
+      asm volatile("" : "+v"(lane1));
+    }
 #pragma unroll
     for (int s = 0; s < 4 * MAXW; s++) {
       const int f = (sp.w0 + min(s >> 2, max(sp.nw - 1, 0))) * 4 + (s & 3);
-      px[s] = ld_ch8(X, (uint32_t)(f * 1024 + lane8));
-      qx[s] = ld_ch8(X, (uint32_t)(f * 1024 + 512 + lane8));
+      px[s] = ld_ch8(X, (uint32_t)(f * 1024 + lane0));
+      if (RT > 1) qx[s] = ld_ch8(X, (uint32_t)(f * 1024 + 512 + lane1));
     }
     bool ok = true;
 #pragma unroll
     for (int s = 0; s < 4 * MAXW; s++) {
       ok &= fresh8(px[s]);
-      ok &= fresh8(qx[s]);
+      if (RT > 1) ok &= fresh8(qx[s]);
     }
     return ok;
   }
-  __device__ __forceinline__ void compute(Span sp) {
+  __device__ __forceinline__ void compute(Span sp) { compute(sp, px, qx); }
+  __device__ __forceinline__ void compute(Span sp, const half8 (&p)[4 * MAXW], const half8 (&q)[4 * MAXW]) {
 #pragma unroll
-    for (int r = 0; r < 16; r++) { c0[r] = 0.f; c1[r] = 0.f; }
+    for (int r = 0; r < 16; r++) { c0[r] = 0.f; if (RT > 1) c1[r] = 0.f; }
 #pragma unroll
     for (int s = 0; s < 4 * MAXW; s++) {
-      if ((s >> 2) < sp.nw) {
-        c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(px[s], w[s], c0, 0, 0, 0);
-        c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(qx[s], w[s], c1, 0, 0, 0);
+      if ((s >> 2) < sp.nw) {  // wave-uniform: surplus windows contribute nothing
+        c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(p[s], w[s], c0, 0, 0, 0);
+        if (RT > 1) c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(q[s], w[s], c1, 0, 0, 0);
       }
     }
   }
-  // this wave's partial into red[wave] ([64 rows][32 columns])
-  __device__ __forceinline__ void to_lds(float (*red)[64][32]) const {
+  // this wave's partial into red[wave] ([64 rows][32 columns], the eights of
+  // rows that hold a row below nb)
+  __device__ __forceinline__ void to_lds(float (*red)[64][32], int nb) const {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, col = lane & 31;
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int t = 8 * (r >> 2) + 4 * h + (r & 3);
-      red[wave][t][col] = c0[r];
-      red[wave][t + 32][col] = c1[r];
+    for (int e = 0; e < 4; e++) {
+      if (RT > 1 || 8 * e < nb) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          red[wave][8 * e + 4 * h + r][col] = c0[4 * e + r];
+          if (RT == 3) red[wave][32 + 8 * e + 4 * h + r][col] = c1[4 * e + r];
+        }
+      }
+      if (RT == 2 && 32 + 8 * e < nb) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[wave][32 + 8 * e + 4 * h + r][col] = c1[4 * e + r];
+      }
     }
   }
 };
+
+constexpr int kTailWaves = 16;
 
 // element pair i (of 1024) of a 64 x 32 tile: row i / 16, columns 2 (i % 16), +1
 __device__ __forceinline__ float2 sum_waves(float (*red)[64][32], int w0, int w1) {
@@ -225,19 +241,22 @@ __device__ __forceinline__ void st_frag2(half_t* X, int t, int k, float a, float
 }
 
 // This thread's element pair of a 64 x 32 tile of column group cg: row
-// tid / 16, columns 32 cg + 2 (tid % 16), +1; its index in x [64][D].
-__device__ __forceinline__ int x_index(int cg, int D) {
-  return (threadIdx.x >> 4) * D + cg * 32 + (threadIdx.x & 15) * 2;
+// tid / 16 (at most nb - 1), columns 32 cg + 2 (tid % 16), +1; its index in
+// x [64][D].
+__device__ __forceinline__ int x_index(int cg, int D, int nb) {
+  return min((int)threadIdx.x >> 4, nb - 1) * D + cg * 32 + (threadIdx.x & 15) * 2;
 }
 
 // Residual epilogue of column group cg (Wo, W2): xv (this thread's element
 // pair of x[:, cg], loaded before the GEMM) += acc and is stored; ssq[cg][t] = sum
 // over the group's 32 columns of the new x^2; xg = fp16(x * gain) fragments
-// for the consumer.
-__device__ void resid_epilogue(float2 acc, float2 xv, int cg, float* x, int D, float* ssq, half_t* xg,
-                               const float* gain) {
+// for the consumer.  Rows below nb.
+__device__ void resid_epilogue(float (*red)[64][32], float2 xv, int cg, float* x, int D, float* ssq, half_t* xg,
+                               const float* gain, int nb) {
   const int row = threadIdx.x >> 4, c = cg * 32 + (threadIdx.x & 15) * 2;
-  const uint32_t xi = (uint32_t)x_index(cg, D);
+  if (row >= nb) return;
+  const float2 acc = sum_waves(red, 0, kTailWaves);
+  const uint32_t xi = (uint32_t)x_index(cg, D, nb);
   const __amdgpu_buffer_rsrc_t rx = rsrc(x);
   xv.x += acc.x;
   xv.y += acc.y;
@@ -248,6 +267,13 @@ __device__ void resid_epilogue(float2 acc, float2 xv, int cg, float* x, int D, f
   for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o, 64);  // the row's 16 threads
   if ((threadIdx.x & 15) == 0) st_c1(ssq, (uint32_t)(cg * 64 + row), ss);
   st_frag2(xg, row, c, xv.x * gain[c], xv.y * gain[c + 1]);
+}
+
+// element t of the column groups' sums of squares [ncg][64] (t < nss = 64 ncg,
+// else the last), its row at most nb - 1
+__device__ __forceinline__ int ssq_index(int t, int nss, int nb) {
+  const int e = min(t, nss - 1);
+  return e - max(e % kDecRows - (nb - 1), 0);
 }
 
 // 1 / rms of row `row` from the ncg <= 32 column-group sums of squares: all
@@ -261,8 +287,6 @@ __device__ __forceinline__ float rr_of(const float* ssq, int ncg, int row, int D
   for (int g = 0; g < 32; g++) s += g < ncg ? v[g] : 0.f;
   return 1.0f / sqrtf(s / (float)D + 1e-5f);
 }
-
-constexpr int kTailWaves = 16;
 
 // Device-coherent loads of two floats per thread, base[e0] and base[e1],
 // straight into LDS (buffer_load ... lds), so that no register is held while
@@ -289,8 +313,8 @@ __device__ __forceinline__ void two_to_lds(const float* base, uint32_t e0, uint3
 }
 // This thread's x element pair of column group cg (x_index) -> xs[0][tid],
 // xs[1][tid].
-__device__ __forceinline__ void x_to_lds(const float* x, int cg, int D, float (*xs)[64 * kTailWaves]) {
-  const uint32_t e = (uint32_t)x_index(cg, D);
+__device__ __forceinline__ void x_to_lds(const float* x, int cg, int D, int nb, float (*xs)[64 * kTailWaves]) {
+  const uint32_t e = (uint32_t)x_index(cg, D, nb);
   two_to_lds(x, e, e + 1, lds_rows(xs, 0), lds_rows(xs, 1));
 }
 
@@ -315,7 +339,14 @@ union TailLds {
 
 // GA > 0 (data-polling form only): the launch also holds the next layer's
 // attention for G = GA query heads per kv head (TailArgs::b_att).
-template <bool POLL, int GA>
+// RT: row tiles of 32.  One (nb <= 32 sequences) reads, computes and writes
+// the nb rows alone: every phase waits for its whole input to pass through
+// the shared level, 98 KB per W1|W3 block at 64 rows of 768, and for the sum
+// of 16 waves' tiles in LDS.  A step of 12 such layers, 3 sequences at
+// position 192..256: 356 us with all 64 rows, 264 with 3; 16 at 1024: 390,
+// 309.  Two do so too (47 at 1024: 424, 402), and three are two whose
+// nb = 64 is a constant.
+template <bool POLL, int GA, int RT>
 __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
   __shared__ TailLds lds;
   auto& red = lds.c.red;
@@ -325,6 +356,7 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
   auto& wfail = lds.c.wfail;
   if (__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;  // an earlier wait failed
   const int D = a.D, H = a.H, N1 = a.N1, ncg = D / 32, npair = H / 32;
+  const int nb = RT > 2 ? kDecRows : a.nb;  // rows read and written
   const int nwd = D / 64, nwh = H / 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: window offsets in SGPRs
   const unsigned E = (unsigned)(*a.gstep) * (unsigned)a.L + (unsigned)a.layer + 1u;
@@ -334,13 +366,19 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
   TailSet S{};
   if constexpr (POLL) {
     S = tail_set(a.sets[E & 1], D, H, N1);
-    // the other set back to stale for the next use: its readers belong to
-    // the previous launch, which has finished
-    const __amdgpu_buffer_rsrc_t ro = rsrc(a.sets[(E & 1) ^ 1]);
-    const u32x4v st = {kTailStale, kTailStale, kTailStale, kTailStale};
-    const uint32_t n16 = (uint32_t)(tail_set_bytes(D, H, N1) / 16);
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n16; k += gridDim.x * blockDim.x)
-      __builtin_amdgcn_raw_buffer_store_b128(st, ro, k * 16u, 0, kSc1);
+    // The other set back to stale (every row, whatever nb) for the next use:
+    // its readers belong to the previous launch, which has finished.  A store
+    // ahead of a block's own loads is waited for with them, so the blocks
+    // that wait longest do it (W2 on; by every block, Wo's included, a step
+    // of 64 sequences took 491 us against 483).
+    const int r0 = a.b_wo + a.b_13, nr = a.b_w2 + a.b_q + 1, rb = (int)blockIdx.x - r0;
+    if (rb >= 0 && rb < nr) {
+      const __amdgpu_buffer_rsrc_t ro = rsrc(a.sets[(E & 1) ^ 1]);
+      const u32x4v st = {kTailStale, kTailStale, kTailStale, kTailStale};
+      const uint32_t n16 = (uint32_t)(tail_set_bytes(D, H, N1) / 16);
+      for (uint32_t k = rb * blockDim.x + threadIdx.x; k < n16; k += nr * blockDim.x)
+        __builtin_amdgcn_raw_buffer_store_b128(st, ro, k * 16u, 0, kSc1);
+    }
   }
   int b = blockIdx.x;
 
@@ -348,17 +386,17 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
     const int cg = b;
     // x was last written before this launch (by the previous layer's W2 or the
     // embedding): a plain load, issued with the weights
-    float2 xv = *reinterpret_cast<const float2*>(a.x + x_index(cg, D));
+    float2 xv = *reinterpret_cast<const float2*>(a.x + x_index(cg, D, nb));
     const Span sp = wave_span<1>(nwd, kTailWaves, wave);
-    WaveGemm<1> g;
+    WaveGemm<1, RT> g;
     g.load_w(a.wo, cg, nwd, sp);
-    g.mma(a.att, sp, false);  // the attention kernel finished before this launch
-    g.to_lds(red);
+    g.mma(a.att, sp, false, nb);  // the attention kernel finished before this launch
+    g.to_lds(red, nb);
     __syncthreads();
     if constexpr (POLL) {  // x after Wo goes to x_mid, for this group's W2 block
-      resid_epilogue(sum_waves(red, 0, kTailWaves), xv, cg, S.x_mid, D, S.ssq_wo, S.xg_ffn, a.g_ffn);
+      resid_epilogue(red, xv, cg, S.x_mid, D, S.ssq_wo, S.xg_ffn, a.g_ffn, nb);
     } else {
-      resid_epilogue(sum_waves(red, 0, kTailWaves), xv, cg, a.x, D, a.ssq_wo, a.xg_ffn, a.g_ffn);
+      resid_epilogue(red, xv, cg, a.x, D, a.ssq_wo, a.xg_ffn, a.g_ffn, nb);
       publish(done_wo);
     }
     return;
@@ -368,7 +406,7 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
     // pair p: W1 rows of hidden units 32 p.. (group 2 p) on waves 0-7, W3 (2 p + 1) on 8-15
     const int pr = b, half = wave >> 3;
     const Span sp = wave_span<2>(nwd, kTailWaves / 2, wave & 7);
-    WaveGemm<2> g;
+    WaveGemm<2, RT> g;
     g.load_w(a.w13, 2 * pr + half, nwd, sp);
     // the residual's column-group sums of squares (ncg * 64 <= 2 per thread),
     // in flight with the activations
@@ -381,8 +419,8 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
       bool ok = false;
       for (unsigned r = 0; a.spin_limit != 0; r++) {
         asm volatile("" ::: "memory");
-        two_to_lds(S.ssq_wo, (uint32_t)min(t0, nss - 1), (uint32_t)min(t1, nss - 1), l0, l1);
-        bool f = g.load_x(S.xg_ffn, sp);
+        two_to_lds(S.ssq_wo, (uint32_t)ssq_index(t0, nss, nb), (uint32_t)ssq_index(t1, nss, nb), l0, l1);
+        bool f = g.load_x(S.xg_ffn, sp, nb);
         drain_stores();  // the LDS loads above
         f &= fresh(ssq_f[0][threadIdx.x]);
         f &= fresh(ssq_f[1][threadIdx.x]);
@@ -391,27 +429,29 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
       }
       wave_outcome(ok, a.err, wfail);
       g.compute(sp);
-      g.to_lds(red);
+      g.to_lds(red, nb);
       __syncthreads();
       if (any_failed(wfail)) return;
     } else {
       if (!wait_count(done_wo, (unsigned)ncg * E, a.spin_limit, a.err, &sh)) return;  // x, its sums of squares, xg_ffn
       const float s0 = t0 < nss ? ld_c1(a.ssq_wo, (uint32_t)t0) : 0.f;
       const float s1 = t1 < nss ? ld_c1(a.ssq_wo, (uint32_t)t1) : 0.f;
-      g.mma(a.xg_ffn, sp, true);
-      g.to_lds(red);
+      g.mma(a.xg_ffn, sp, true, nb);
+      g.to_lds(red, nb);
       if (t0 < nss) ssq_s[t0 / kDecRows][t0 % kDecRows] = s0;
       if (t1 < nss) ssq_s[t1 / kDecRows][t1 % kDecRows] = s1;
       __syncthreads();
     }
-    const float2 h1 = sum_waves(red, 0, kTailWaves / 2), h3 = sum_waves(red, kTailWaves / 2, kTailWaves);
     const int row = threadIdx.x >> 4, c = (threadIdx.x & 15) * 2;
-    float ss = 0.f;
-    for (int q = 0; q < ncg; q++) ss += ssq_s[q][row];
-    const float rr = 1.0f / sqrtf(ss / (float)D + 1e-5f);
-    const float u0 = h1.x * rr, u1 = h1.y * rr;
-    st_frag2(POLL ? S.gate : a.gate, row, 32 * pr + c, u0 / (1.0f + __expf(-u0)) * (h3.x * rr),
-             u1 / (1.0f + __expf(-u1)) * (h3.y * rr));
+    if (row < nb) {
+      const float2 h1 = sum_waves(red, 0, kTailWaves / 2), h3 = sum_waves(red, kTailWaves / 2, kTailWaves);
+      float ss = 0.f;
+      for (int q = 0; q < ncg; q++) ss += ssq_s[q][row];
+      const float rr = 1.0f / sqrtf(ss / (float)D + 1e-5f);
+      const float u0 = h1.x * rr, u1 = h1.y * rr;
+      st_frag2(POLL ? S.gate : a.gate, row, 32 * pr + c, u0 / (1.0f + __expf(-u0)) * (h3.x * rr),
+               u1 / (1.0f + __expf(-u1)) * (h3.y * rr));
+    }
     if constexpr (!POLL) publish(done_13);
     return;
   }
@@ -419,18 +459,18 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
   if (b < a.b_w2) {  // ---- W2: x += W2 gate -----------------------------------
     const int cg = b;
     const Span sp = wave_span<2>(nwh, kTailWaves, wave);
-    WaveGemm<2> g;
+    WaveGemm<2, RT> g;
     g.load_w(a.w2, cg, nwh, sp);
     if constexpr (POLL) {
       // x after Wo (x_mid, from this group's Wo block) in the same rounds as
       // the activations, straight into LDS
-      const uint32_t xm = (uint32_t)x_index(cg, D);
+      const uint32_t xm = (uint32_t)x_index(cg, D, nb);
       const unsigned l0 = lds_rows(xs, 0), l1 = lds_rows(xs, 1);
       bool ok = false;
       for (unsigned r = 0; a.spin_limit != 0; r++) {
         asm volatile("" ::: "memory");
         two_to_lds(S.x_mid, xm, xm + 1, l0, l1);
-        bool f = g.load_x(S.gate, sp);
+        bool f = g.load_x(S.gate, sp, nb);
         drain_stores();  // the LDS loads above
         f &= fresh(xs[0][threadIdx.x]);
         f &= fresh(xs[1][threadIdx.x]);
@@ -439,25 +479,24 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
       }
       wave_outcome(ok, a.err, wfail);
       g.compute(sp);
-      g.to_lds(red);
+      g.to_lds(red, nb);
       __syncthreads();
       if (any_failed(wfail)) return;
     } else {
       // done_13 implies done_wo: x (written by the Wo block of this group) is
       // read device-coherent, in flight with the activations
       if (!wait_count(done_13, (unsigned)npair * E, a.spin_limit, a.err, &sh)) return;
-      x_to_lds(a.x, cg, D, xs);
-      g.mma(a.gate, sp, true);
-      g.to_lds(red);
+      x_to_lds(a.x, cg, D, nb, xs);
+      g.mma(a.gate, sp, true, nb);
+      g.to_lds(red, nb);
       drain_stores();  // (also the loads: x_to_lds is not in the compiler's count)
       __syncthreads();
     }
     const float2 xv = make_float2(xs[0][threadIdx.x], xs[1][threadIdx.x]);
     if constexpr (POLL) {  // the last layer's output is for the classifier (after this launch)
-      resid_epilogue(sum_waves(red, 0, kTailWaves), xv, cg, a.x, D, S.ssq_w2, a.b_q ? S.xg_next : a.xg_next,
-                     a.g_next);
+      resid_epilogue(red, xv, cg, a.x, D, S.ssq_w2, a.b_q ? S.xg_next : a.xg_next, a.g_next, nb);
     } else {
-      resid_epilogue(sum_waves(red, 0, kTailWaves), xv, cg, a.x, D, a.ssq_w2, a.xg_next, a.g_next);
+      resid_epilogue(red, xv, cg, a.x, D, a.ssq_w2, a.xg_next, a.g_next, nb);
       publish(done_w2);
     }
     return;
@@ -466,28 +505,29 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
   if (b < a.b_q) {  // ---- next layer's QKV (finished by the attention) ----------------
     const int cg = b;
     const Span sp = wave_span<1>(nwd, kTailWaves, wave);
-    WaveGemm<1> g;
+    WaveGemm<1, RT> g;
     g.load_w(a.wqkv_next, cg, nwd, sp);
     if constexpr (POLL) {
       bool ok = false;
       for (unsigned r = 0; a.spin_limit != 0; r++) {
         asm volatile("" ::: "memory");
-        if (__all(g.load_x(S.xg_next, sp))) { ok = true; break; }
+        if (__all(g.load_x(S.xg_next, sp, nb))) { ok = true; break; }
         if (give_up(r, a.spin_limit, a.err)) break;
       }
       wave_outcome(ok, a.err, wfail);
       g.compute(sp);
-      g.to_lds(red);
+      g.to_lds(red, nb);
       __syncthreads();
       if (any_failed(wfail)) return;
     } else {
       if (!wait_count(done_w2, (unsigned)ncg * E, a.spin_limit, a.err, &sh)) return;
-      g.mma(a.xg_next, sp, true);
-      g.to_lds(red);
+      g.mma(a.xg_next, sp, true, nb);
+      g.to_lds(red, nb);
       __syncthreads();
     }
-    const float2 v = sum_waves(red, 0, kTailWaves);
     const int row = threadIdx.x >> 4, c = cg * 32 + (threadIdx.x & 15) * 2;
+    if (row >= nb) return;
+    const float2 v = sum_waves(red, 0, kTailWaves);
     if (POLL && a.b_att) {  // for the attention blocks of this launch
       st_c1(S.p_q, (uint32_t)(row * N1 + c), v.x);
       st_c1(S.p_q, (uint32_t)(row * N1 + c + 1), v.y);
@@ -532,7 +572,7 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
       bool f = true;
 #pragma unroll
       for (int q = 0; q < 32; q++) {
-        v[q] = ld_c1(S.ssq_w2, (uint32_t)(min(q, ncg - 1) * 64 + row));
+        v[q] = ld_c1(S.ssq_w2, (uint32_t)(min(q, ncg - 1) * 64 + min(row, nb - 1)));
         f &= fresh(v[q]);
       }
       if (__all(f)) { ok = true; break; }
@@ -546,6 +586,7 @@ __global__ __launch_bounds__(64 * kTailWaves) void tail_kernel(TailArgs a) {
 #pragma unroll
     for (int q = 0; q < 32; q++) ss += q < ncg ? v[q] : 0.f;
     const float r = 1.0f / sqrtf(ss / (float)D + 1e-5f);
+    if (row >= nb) return;
     if (a.b_att) st_c1(S.rr, (uint32_t)row, r);
     else a.rr_next[row] = r;
   } else {
@@ -593,6 +634,7 @@ __global__ __launch_bounds__(256) void row_xg_kernel(float* x, half_t* xg, float
 hipError_t dec_tail(const TailArgs& a, hipStream_t s) {
   // one window per wave for K = D (<= 16 windows), two for K = H (<= 32)
   if (a.D % 64 || a.D > 1024 || a.H % 64 || a.H > 2048 || a.N1 % 32) return hipErrorInvalidValue;
+  if (a.nb < 1 || a.nb > kDecRows) return hipErrorInvalidValue;
   if (a.b_wo != a.D / 32 || a.b_13 != a.H / 32 || a.b_w2 != a.D / 32 || (a.b_q && a.b_q != a.N1 / 32))
     return hipErrorInvalidValue;
   if (a.poll && (!a.sets[0] || !a.sets[1])) return hipErrorInvalidValue;
@@ -605,14 +647,19 @@ hipError_t dec_tail(const TailArgs& a, hipStream_t s) {
   }
   const int blocks = a.b_wo + a.b_13 + a.b_w2 + a.b_q + 1 + a.b_att;
   const dim3 g(blocks), t(64 * kTailWaves);
+#define TAIL(GA_)                                                                                   \
+  if (a.nb <= 32) hipLaunchKernelGGL((tail_kernel<true, GA_, 1>), g, t, 0, s, a);                   \
+  else if (a.nb < kDecRows) hipLaunchKernelGGL((tail_kernel<true, GA_, 2>), g, t, 0, s, a);         \
+  else hipLaunchKernelGGL((tail_kernel<true, GA_, 3>), g, t, 0, s, a);
   switch (a.poll ? ga + 1 : 0) {
-    case 0: hipLaunchKernelGGL((tail_kernel<false, 0>), g, t, 0, s, a); break;
-    case 1: hipLaunchKernelGGL((tail_kernel<true, 0>), g, t, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((tail_kernel<true, 1>), g, t, 0, s, a); break;
-    case 3: hipLaunchKernelGGL((tail_kernel<true, 2>), g, t, 0, s, a); break;
-    case 4: hipLaunchKernelGGL((tail_kernel<true, 3>), g, t, 0, s, a); break;
-    default: hipLaunchKernelGGL((tail_kernel<true, 4>), g, t, 0, s, a); break;
+    case 0: hipLaunchKernelGGL((tail_kernel<false, 0, 3>), g, t, 0, s, a); break;
+    case 1: TAIL(0); break;
+    case 2: TAIL(1); break;
+    case 3: TAIL(2); break;
+    case 4: TAIL(3); break;
+    default: TAIL(4); break;
   }
+#undef TAIL
   return hipGetLastError();
 }
 
@@ -624,12 +671,13 @@ int dec_tail_blocks_per_cu() {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 64 * kTailWaves, 0) != hipSuccess) n = 0;
     m = n < m ? n : m;
   };
-  occ((const void*)tail_kernel<false, 0>);
-  occ((const void*)tail_kernel<true, 0>);
-  occ((const void*)tail_kernel<true, 1>);
-  occ((const void*)tail_kernel<true, 2>);
-  occ((const void*)tail_kernel<true, 3>);
-  occ((const void*)tail_kernel<true, 4>);
+  occ((const void*)tail_kernel<false, 0, 3>);
+#define TAIL(GA_)                              \
+  occ((const void*)tail_kernel<true, GA_, 1>); \
+  occ((const void*)tail_kernel<true, GA_, 2>); \
+  occ((const void*)tail_kernel<true, GA_, 3>);
+  TAIL(0) TAIL(1) TAIL(2) TAIL(3) TAIL(4)
+#undef TAIL
   return m;
 }
 

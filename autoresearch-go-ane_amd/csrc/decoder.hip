@@ -405,7 +405,7 @@ int enqueue_step_tail(ane_decoder* d, float* logits, uint16_t* hist) {
     t.p_q = d->kpart;
     t.ssq_wo = d->ssq_wo; t.ssq_w2 = d->ssq_w2; t.sync = d->sync; t.gstep = d->ctr_d + 2; t.err = d->err_d;
     t.spin_limit = d->tail_spin;
-    t.D = D; t.H = H; t.N1 = N1; t.layer = l; t.L = L;
+    t.D = D; t.H = H; t.N1 = N1; t.layer = l; t.L = L; t.nb = nb;
     t.b_wo = D / 32; t.b_13 = H / 32; t.b_w2 = D / 32; t.b_q = last ? 0 : N1 / 32;
     t.poll = d->tail_poll ? 1 : 0;
     t.sets[0] = d->tail_sets;

@@ -258,6 +258,33 @@ def test_full_batch_of_64_every_sequence(heads, kv_heads, tail, monkeypatch):
     _check_choice(gen, g_lg[:, 1:])
 
 
+@pytest.mark.parametrize("tail", ["2", "1"])
+def test_batches_of_every_row_form_in_turn(tail, monkeypatch):
+    """One decoder through batches on both sides of the chain's row forms
+    (one 32-row tile, two, all 64 rows), smaller after larger and larger
+    after smaller: no row of an earlier batch is read, and every buffer set
+    starts unwritten.  Two layers, so that the second layer's attention runs
+    in the first's launch; forced steps of every sequence against the oracle."""
+    monkeypatch.setenv("ANE_DEC_TAIL", tail)
+    cfg = ane.tiny_decode(heads=6, kv_heads=2, dim=384, layers=2)
+    plen, nsteps = 64, 2
+    p, prefix = _setup(cfg, 64, plen, 83)
+    forced = np.random.default_rng(84).integers(0, cfg.vocab, (64, nsteps)).astype(np.uint16)
+    _, ref = oracle.decode(cfg, p, prefix, nsteps, forced=forced, want_logits=True)
+    dec = ane.Decoder(cfg, p, max_batch=64, max_ctx=128)
+    try:
+        for nseq in (64, 1, 33, 8, 63, 32, 9, 64, 31):
+            dec.Prefill(prefix[:nseq])
+            for i in range(nsteps):
+                tok, lg = dec.Step(forced[:nseq, i], want_logits=True)
+                err = np.abs(lg - ref[:nseq, i + 1]).max()
+                assert err <= TOL, (nseq, i, err)
+                np.testing.assert_array_equal(tok, lg.argmax(-1))
+        assert dec.FusedChain() == 1
+    finally:
+        dec.Close()
+
+
 @pytest.mark.parametrize("tail,form", [("2", None), ("2", "wide"), ("1", None)])
 def test_fused_chain_wait_timeout_falls_back(tail, form, monkeypatch):
     """A dependency wait of the fused layer kernel that times out does not
