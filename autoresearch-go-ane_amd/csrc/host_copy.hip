@@ -11,6 +11,15 @@ namespace ane {
 namespace {
 inline void pause_cpu() { __builtin_ia32_pause(); }
 
+// First touch of a page about to be written: a write that changes nothing.
+// One locked instruction, so that a copy which another thread has meanwhile
+// made to this byte stays (a load and a store could put the old byte back);
+// in asm, as the compiler turns an atomic "or 0" into a fence and a load,
+// which gives the page no memory of its own.
+inline void touch_page(void* p) {
+  asm volatile("lock orb $0, %0" : "+m"(*(char*)p) : : "memory", "cc");
+}
+
 std::mutex g_pools_mu;
 constexpr int kMaxDevices = 64;
 constexpr uintptr_t kPage = (uintptr_t)2 << 20;  // a transparent huge page
@@ -107,9 +116,8 @@ bool HostPool::step() {
     if (head_.compare_exchange_weak(h, h + 1, std::memory_order_acq_rel)) {
       if (src) {
         memcpy(dst, src, n);
-      } else {  // first touch of a page about to be written
-        volatile char* c = (volatile char*)dst;
-        *c = *c;
+      } else {
+        touch_page(dst);
       }
       left->fetch_sub(1, std::memory_order_release);
       return true;
