@@ -171,12 +171,15 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
 // that return results to their caller.  hipStreamSynchronize may block the
 // thread until an interrupt wakes it, tens of microseconds after the GPU has
 // finished; polling returns within a few.  ANE_SPIN_WAIT=0 blocks instead.
-inline hipError_t stream_wait(hipStream_t s) {
+inline bool spin_waits() {
   static const bool spin = [] {
     const char* f = getenv("ANE_SPIN_WAIT");
     return !f || atoi(f) != 0;
   }();
-  if (!spin) return hipStreamSynchronize(s);
+  return spin;
+}
+inline hipError_t stream_wait(hipStream_t s) {
+  if (!spin_waits()) return hipStreamSynchronize(s);
   hipError_t r;
   while ((r = hipStreamQuery(s)) == hipErrorNotReady) {
   }

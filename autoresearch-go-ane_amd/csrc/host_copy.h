@@ -35,6 +35,9 @@ class HostPool {
   static constexpr int kThreads = 6;
   // below this a copy is left to hipMemcpyAsync: waking the threads costs more
   static constexpr size_t kMinBytes = (size_t)256 << 10;
+  // how long a thread looks for pieces before it sleeps: past the gap between
+  // two slots' arrivals (75 us on the link), far below a wait for kernels
+  static constexpr int kIdleUs = 300;
 
   ~HostPool();
 
@@ -60,8 +63,7 @@ class HostPool {
   void run();                    // a thread's loop
   bool step();                   // copies one queued piece; false if there is none
   void push(void* dst, const void* src, size_t n, std::atomic<int>* left);
-  void wake();
-  void rest();
+  void wake();                   // sleeping threads look for pieces again, for kIdleUs at least
 
   static constexpr int kRing = 256;
   std::mutex use_;               // held by the HostCopy in hand
@@ -73,7 +75,10 @@ class HostPool {
   std::atomic<unsigned> head_{0}, tail_{0};
   std::mutex mu_;
   std::condition_variable cv_;
-  std::atomic<bool> awake_{false}, stop_{false};
+  std::atomic<int> asleep_{0};
+  std::atomic<unsigned> calls_{0};  // wake()s so far
+  std::atomic<bool> stop_{false};
+  hipEvent_t ahead_ = nullptr;      // after what a call's first copy to the host waits for
   std::vector<std::thread> threads_;
 };
 
@@ -100,6 +105,7 @@ class HostCopy {
   hipError_t pass(HostPool::Slot* s);             // a device-to-host slot whose event has passed: hand out its pieces
   void drain(std::atomic<int>* left);             // copy pieces until *left is 0
   hipError_t pass_first();
+  hipError_t wait(hipEvent_t ev);                 // copies pieces meanwhile
   void split(char* dst, const char* src, size_t n, std::atomic<int>* left);
   std::shared_ptr<HostPool>* handle_;
   int device_;
@@ -108,6 +114,8 @@ class HostCopy {
   bool busy_ = false;                             // another thread has the pool: not asked again
   int pending_[HostPool::kSlots];                 // slots queued to the host: n_pending_ from first_, oldest first
   int first_ = 0, n_pending_ = 0;
+  bool down_ = false;                             // p_->ahead_ is recorded, by the first copy to the host ...
+  bool ahead_ = false;                            // ... and not yet waited for
 };
 
 }  // namespace ane

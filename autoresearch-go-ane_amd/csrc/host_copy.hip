@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 
 namespace ane {
 
@@ -58,13 +59,17 @@ bool HostPool::init(int device) {
     (void)hipGetLastError();
     return false;
   }
+  auto event = [](hipEvent_t* ev) {
+    if (hipEventCreateWithFlags(ev, hipEventDisableTiming | (spin_waits() ? 0 : hipEventBlockingSync)) == hipSuccess)
+      return true;
+    *ev = nullptr;
+    (void)hipGetLastError();
+    return false;
+  };
+  if (!event(&ahead_)) return false;
   for (int i = 0; i < kSlots; i++) {
     slots_[i].mem = mem_ + i * kSlotBytes;
-    if (hipEventCreateWithFlags(&slots_[i].ev, hipEventDisableTiming) != hipSuccess) {
-      slots_[i].ev = nullptr;
-      (void)hipGetLastError();
-      return false;
-    }
+    if (!event(&slots_[i].ev)) return false;
   }
   try {
     const unsigned hw = std::thread::hardware_concurrency();
@@ -88,20 +93,35 @@ HostPool::~HostPool() {
       if (s.in_flight) (void)hipEventSynchronize(s.ev);
       (void)hipEventDestroy(s.ev);
     }
+  if (ahead_) (void)hipEventDestroy(ahead_);
   if (mem_) (void)hipHostFree(mem_);
 }
 
+// Looks for pieces while there are any and for kIdleUs after the last one or
+// the last wake(), then sleeps: a call that waits for kernels keeps no thread busy.
 void HostPool::run() {
+  using clock = std::chrono::steady_clock;
+  unsigned seen = 0;
   for (;;) {
+    for (clock::time_point since = clock::now();;) {
+      const unsigned c = calls_.load(std::memory_order_acquire);
+      const bool worked = step();
+      if (worked || c != seen) {
+        seen = c;
+        since = clock::now();
+        continue;
+      }
+      if (stop_ || clock::now() - since > std::chrono::microseconds(kIdleUs)) break;
+      for (int i = 0; i < 32; i++) pause_cpu();
+    }
     {
       std::unique_lock<std::mutex> lk(mu_);
-      cv_.wait(lk, [this] { return stop_ || awake_; });
+      asleep_.fetch_add(1);
+      cv_.wait(lk, [&] { return stop_ || calls_.load() != seen; });
+      asleep_.fetch_sub(1);
       if (stop_) return;
     }
     cv_.notify_one();  // the next sleeper (the caller wakes one thread, not all: ~12 us each)
-    while (awake_.load(std::memory_order_acquire) && !stop_)
-      if (!step())
-        for (int i = 0; i < 32; i++) pause_cpu();
   }
 }
 
@@ -137,14 +157,14 @@ void HostPool::push(void* dst, const void* src, size_t n, std::atomic<int>* left
   tail_.store(t + 1, std::memory_order_release);
 }
 
+// A thread counts itself asleep before it reads calls_ for the last time, and
+// here calls_ changes before asleep_ is read: one of the two sees the other.
 void HostPool::wake() {
-  {
-    std::lock_guard<std::mutex> lk(mu_);
-    awake_ = true;
-  }
+  calls_.fetch_add(1);
+  if (asleep_.load() == 0) return;
+  { std::lock_guard<std::mutex> lk(mu_); }  // (a thread between its read and its wait)
   cv_.notify_one();
 }
-void HostPool::rest() { awake_.store(false, std::memory_order_release); }
 
 // ---- one call's copies ---------------------------------------------------------
 
@@ -162,7 +182,6 @@ bool HostCopy::take(const void* host, size_t n) {
     return false;
   }
   p_ = handle_->get();
-  p_->wake();
   return true;
 }
 
@@ -176,12 +195,27 @@ void HostCopy::split(char* dst, const char* src, size_t n, std::atomic<int>* lef
   left->fetch_add(k, std::memory_order_relaxed);
   for (size_t o = 0; o < n; o += HostPool::kTaskBytes)
     p_->push(dst + o, src + o, std::min(HostPool::kTaskBytes, n - o), left);
+  p_->wake();
+}
+
+hipError_t HostCopy::wait(hipEvent_t ev) {
+  hipError_t h;
+  while ((h = hipEventQuery(ev)) == hipErrorNotReady) {
+    if (p_->step()) continue;
+    if (!spin_waits()) return hipEventSynchronize(ev);
+    pause_cpu();
+  }
+  return h;
 }
 
 hipError_t HostCopy::pass(HostPool::Slot* s) {
-  hipError_t h;
-  while ((h = hipEventQuery(s->ev)) == hipErrorNotReady)
-    if (!p_->step()) pause_cpu();
+  hipError_t h = hipSuccess;
+  if (ahead_) {  // the link starts now: threads that slept through the kernels wake meanwhile
+    h = wait(p_->ahead_);
+    ahead_ = false;
+    p_->wake();
+  }
+  if (h == hipSuccess) h = wait(s->ev);
   s->in_flight = false;
   if (h == hipSuccess && s->host) split(s->host, s->mem, s->n, &s->left);
   s->host = nullptr;
@@ -226,16 +260,23 @@ hipError_t HostCopy::up(void* dst, const void* src, size_t n) {
 
 hipError_t HostCopy::down(void* dst, const void* src, size_t n) {
   if (!take(dst, n)) return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st_);
+  if (!down_) {
+    const hipError_t h = hipEventRecord(p_->ahead_, st_);
+    if (h != hipSuccess) return h;
+    down_ = ahead_ = true;
+  }
   // A buffer the caller has just allocated has no pages yet.  Each is touched
   // by one thread before its bytes arrive: left to the copies, several
   // threads would fault the same 2 MB page and each clear one for it.
   const uintptr_t end = (uintptr_t)dst + n;
   uintptr_t touch = n >= 2 * kPage ? (uintptr_t)dst : end;
   auto touch_to = [&](uintptr_t upto) {
+    if (touch >= std::min(upto, end)) return;
     for (; touch < std::min(upto, end); touch = (touch | (kPage - 1)) + 1) {
       p_->touched_.fetch_add(1, std::memory_order_relaxed);
       p_->push((void*)touch, nullptr, 0, &p_->touched_);
     }
+    p_->wake();
   };
   for (size_t o = 0; o < n; o += HostPool::kSlotBytes) {
     const size_t k = std::min(HostPool::kSlotBytes, n - o);
@@ -281,7 +322,6 @@ HostCopy::~HostCopy() {
   }
   for (HostPool::Slot& s : p_->slots_) drain(&s.left);
   drain(&p_->touched_);
-  p_->rest();
   p_->use_.unlock();
 }
 
