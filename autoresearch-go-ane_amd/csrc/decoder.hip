@@ -70,7 +70,7 @@ struct ane_decoder {
   int D = 0, H = 0, NH = 0, NKV = 0, KVD = 0, N1 = 0, L = 0, V = 0, B = 0, C = 0;
   std::string err;
   hipStream_t stream = nullptr;
-  std::shared_ptr<HostPool> host_pool;  // from the first large copy on
+  HostPoolRef host_pool;
   std::vector<void*> allocs;
   std::vector<DecLayerOff> off;
   int64_t off_embed = 0, off_gfinal = 0, nparams = 0;

@@ -225,7 +225,7 @@ static void free_all(ane_engine* e) {
   if (e->stream) (void)hipStreamSynchronize(e->stream);
   for (void* p : e->allocs) (void)hipFree(p);
   e->allocs.clear();
-  e->host_pool.reset();
+  e->host_pool = {};
   if (e->loss_host) (void)hipHostFree(e->loss_host);
   e->loss_host = nullptr;
   for (ProfEvent& pe : e->prof_events) {

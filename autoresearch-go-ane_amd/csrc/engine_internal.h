@@ -119,7 +119,7 @@ struct ane_engine {
   ane_model_cfg cfg{};
   ane_options opt{};
   int device = 0;
-  std::shared_ptr<ane::HostPool> host_pool;  // from the first large copy on
+  ane::HostPoolRef host_pool;
   bool dev_set = false;
   bool closed = false;
   std::string err;

@@ -35,6 +35,11 @@ class HostPool {
   static constexpr int kThreads = 6;
   // below this a copy is left to hipMemcpyAsync: waking the threads costs more
   static constexpr size_t kMinBytes = (size_t)256 << 10;
+  // what an object has to copy before a pool is made for it (one that is
+  // there already is used at once): making it, 32 MB of pinned memory and the
+  // threads, costs about what the pool saves on 8 MB.  Opening and closing a
+  // model of 1.6 MB: 310 us without one, 500 with it
+  static constexpr size_t kMakeBytes = (size_t)8 << 20;
   // how long a thread looks for pieces before it sleeps: past the gap between
   // two slots' arrivals (75 us on the link), far below a wait for kernels
   static constexpr int kIdleUs = 300;
@@ -43,7 +48,7 @@ class HostPool {
 
  private:
   friend class HostCopy;
-  friend std::shared_ptr<HostPool> host_pool(int device);
+  friend std::shared_ptr<HostPool> host_pool(int device, bool make);
   struct Task {  // (read by threads that may then fail to claim it, hence atomic)
     std::atomic<void*> dst;
     std::atomic<const void*> src;
@@ -82,16 +87,23 @@ class HostPool {
   std::vector<std::thread> threads_;
 };
 
-// The current device's pool; null if it cannot be made (then hipMemcpyAsync serves).
-std::shared_ptr<HostPool> host_pool(int device);
+// The device's pool; null if there is none and it is not to be (or cannot be)
+// made: then hipMemcpyAsync serves.
+std::shared_ptr<HostPool> host_pool(int device, bool make);
+
+// An object's hold on its device's pool, and the large copies it had without one.
+struct HostPoolRef {
+  std::shared_ptr<HostPool> pool;
+  size_t bytes = 0;
+};
 
 // The copies of one call, on one stream.  up() returns once the source may be
 // reused; down() queues, and finish() waits until every destination is
 // written.  Copies take their place in the stream's order.
 class HostCopy {
  public:
-  // pool: the caller's handle, filled on the first copy large enough to need it
-  HostCopy(std::shared_ptr<HostPool>* pool, int device, hipStream_t st) : handle_(pool), device_(device), st_(st) {}
+  // ref: the calling object's, filled by the copy from which the pool pays
+  HostCopy(HostPoolRef* ref, int device, hipStream_t st) : ref_(ref), device_(device), st_(st) {}
   ~HostCopy();
   HostCopy(const HostCopy&) = delete;
   HostCopy& operator=(const HostCopy&) = delete;
@@ -107,11 +119,11 @@ class HostCopy {
   hipError_t pass_first();
   hipError_t wait(hipEvent_t ev);                 // copies pieces meanwhile
   void split(char* dst, const char* src, size_t n, std::atomic<int>* left);
-  std::shared_ptr<HostPool>* handle_;
+  HostPoolRef* ref_;
   int device_;
   hipStream_t st_;
   HostPool* p_ = nullptr;                         // locked
-  bool busy_ = false;                             // another thread has the pool: not asked again
+  bool busy_ = false;                             // another thread has the pool, or there is none: not asked again
   int pending_[HostPool::kSlots];                 // slots queued to the host: n_pending_ from first_, oldest first
   int first_ = 0, n_pending_ = 0;
   bool down_ = false;                             // p_->ahead_ is recorded, by the first copy to the host ...

@@ -27,10 +27,11 @@ constexpr uintptr_t kPage = (uintptr_t)2 << 20;  // a transparent huge page
 std::weak_ptr<HostPool> g_pools[kMaxDevices];
 }  // namespace
 
-std::shared_ptr<HostPool> host_pool(int device) {
+std::shared_ptr<HostPool> host_pool(int device, bool make) {
   if (device < 0 || device >= kMaxDevices) return nullptr;
   std::lock_guard<std::mutex> lk(g_pools_mu);
   if (auto p = g_pools[device].lock()) return p;
+  if (!make) return nullptr;
   try {
     std::shared_ptr<HostPool> p(new HostPool());
     if (!p->init(device)) return nullptr;
@@ -176,12 +177,20 @@ bool HostCopy::take(const void* host, size_t n) {
   if (hipPointerGetAttributes(&at, host) != hipSuccess) (void)hipGetLastError();
   else if (at.type != hipMemoryTypeUnregistered) return false;
   if (p_) return true;
-  if (!*handle_) *handle_ = host_pool(device_);
-  if (!*handle_ || !(*handle_)->use_.try_lock()) {
+  if (!ref_->pool) {
+    ref_->bytes = std::min(ref_->bytes + n, HostPool::kMakeBytes);
+    const bool make = ref_->bytes == HostPool::kMakeBytes;
+    ref_->pool = host_pool(device_, make);
+    if (!ref_->pool) {
+      busy_ = make;  // (it cannot be made: not tried again by this call)
+      return false;
+    }
+  }
+  if (!ref_->pool->use_.try_lock()) {
     busy_ = true;
     return false;
   }
-  p_ = handle_->get();
+  p_ = ref_->pool.get();
   return true;
 }
 

@@ -272,7 +272,7 @@ struct ane_moe {
   int D = 0, H = 0, E = 0, TM = 0, RC = 0, T = 0;
   std::string err;
   hipStream_t stream = nullptr;
-  std::shared_ptr<HostPool> host_pool;  // from the first large copy on
+  HostPoolRef host_pool;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::vector<void*> allocs;
   bool params_set = false;

@@ -202,7 +202,7 @@ struct SeamBase {
   hipStream_t st = nullptr;
   std::vector<void*> allocs;
   bool closed = false;
-  std::shared_ptr<HostPool> pool;  // from the first large copy on
+  HostPoolRef pool;
   HostCopy* copies = nullptr;      // those of the call in hand (Copies)
 
   template <typename T>
@@ -221,7 +221,7 @@ struct SeamBase {
     allocs.clear();
     if (st) (void)hipStreamDestroy(st);
     st = nullptr;
-    pool.reset();
+    pool = {};
     closed = true;
   }
   // the device and stream every call of the object uses

@@ -1,9 +1,10 @@
 """Copies between the caller's memory and the device through the pool of
 pinned slots: bit-exact round trips at sizes around a piece, a slot and the
 ring (layer weights set and read back, MoE activations), from several threads
-at once, and after every object that shared the pool is closed; and what the
-pool's threads cost a call that waits for kernels."""
+at once, and after every object that shared the pool is closed; what the pool's
+threads cost a call that waits for kernels, and that small objects make none."""
 import ctypes as C
+import os
 import threading
 import time
 
@@ -24,11 +25,12 @@ def engine(vocab, seed):
     return ane.Open(ane.Options(Config=cfg, Params=p)), p
 
 
-# 64 floats a vocabulary row (and 128 KiB of layer weights): below the pool's
-# least size, at it and past it, around one slot (4 MiB), past the ring of 8
-# slots, past twice that
+# 64 floats a vocabulary row (and 128 KiB of layer weights): below the least
+# size of a copy through the pool, at it and past it, around one slot (4 MiB),
+# past the ring of 8 slots, past twice that
 @pytest.mark.parametrize("vocab", [256, 512, 1024, 15808, 15872, 16384, 131072 + 6400, 65536 * 4 + 64])
 def test_params_round_trip(vocab):
+    other, _ = engine(40000, 3)  # (so that there is a pool, whatever this one's size)
     eng, p = engine(vocab, vocab)
     try:
         for _ in range(2):
@@ -48,6 +50,7 @@ def test_params_round_trip(vocab):
         np.testing.assert_array_equal(gv, v)
     finally:
         eng.Destroy()
+        other.Destroy()
 
 
 def test_threads_share_the_pool():
@@ -95,3 +98,22 @@ def test_threads_sleep_while_a_call_waits_for_kernels():
         assert min(share) < 4.0
     finally:
         eng.Destroy()
+
+
+def test_small_objects_make_no_pool():
+    """A model of 1.5 MB opens and evaluates without the pool's threads (and
+    its 32 MB of pinned memory); one of 10 MB has them, and takes them along."""
+    threads = lambda: len(os.listdir("/proc/self/task"))
+    engine(256, 1)[0].Destroy()  # the runtime's own threads
+    before = threads()
+    cfg = ane.Config(dim=128, hidden=256, heads=2, layers=2, vocab=512, seq=64, arch="llama2")
+    eng = ane.Open(ane.Options(Config=cfg, Params=ane.init_params(cfg, seed=0)))
+    tok, _ = ane.make_tokens(cfg, 1, seed=1)
+    eng.EvalLogits(tok[0])
+    eng.Params()
+    assert threads() == before
+    big, _ = engine(40000, 2)
+    assert threads() > before
+    big.Destroy()
+    assert threads() == before
+    eng.Destroy()
