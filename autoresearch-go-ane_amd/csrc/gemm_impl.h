@@ -152,50 +152,72 @@ __device__ __forceinline__ void wait_vm() {
 // has waited for the loads it needs; LDS reads/writes are drained here.
 __device__ __forceinline__ void barrier_keep_loads() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// cap * tanh(v / cap).  Every VALU instruction per logit costs the classifier
-// of 9984 tokens x 32000 ~10 us, so a lane's values of one column are capped
-// by the shortest form that holds for the largest of them (MA = max |v|, taken
-// over the wave): the Taylor series of tanh to x^7 below cap / 6, to x^13 below
-// 0.45 cap (both within 6e-8 of the value, half an ulp), else per value the
-// latter or 1 - 2 / (e^2x + 1) (within 2.6e-7; NaN and infinities pass through).
-// The cross-entropy GEMM at that size: tanhf 708 us, this 565, no softcap 484.
+// cap * tanh(v / cap) and its derivative, each as exact as tanhf gives them or
+// more (relative to float64, rms / largest, here against tanhf: values below
+// 6.75 of cap 15 2.6e-8 / 6.5e-8 against 4.6e-8 / 1.5e-7, to 30 5.1e-8 / 1.7e-7
+// against 5.6e-8 / 2.0e-7; derivatives at 60 to 90 5.2e-8 against 5.0e-4).
+// Every VALU instruction per logit costs the classifier of 9984 tokens x 32000
+// ~10 us, so three forms by magnitude: the Taylor series of tanh to x^7 below
+// cap / 6, to x^19 below 0.6 cap (both within half an ulp before rounding), else
+// 1 - 2 / (e^2x + 1) with the exponent's rounding error carried into e^2x.  The
+// derivative is 1 - tanh^2 of the series, and 4 r (1 - r) for r = 1 / (e^2x + 1)
+// where that difference would cancel.  NaN stays, infinities give +-cap.
 struct Softcap {
-  float cap, inv, z1, c1, c2, c3, c4, c5, c6;  // series coefficients over powers of v^2
+  float cap, inv, z1, c1, c2, c3, k, klo;  // c: series coefficients over powers of v^2; k + klo = 2 log2(e) / cap
   __device__ __forceinline__ explicit Softcap(float cap_) : cap(cap_), inv(1.f / cap_) {
     z1 = inv * inv;
-    const float z2 = z1 * z1;
     c1 = -1.f / 3.f * z1;
-    c2 = 2.f / 15.f * z2;
-    c3 = -17.f / 315.f * z2 * z1;
-    c4 = 62.f / 2835.f * z2 * z2;
-    c5 = -1382.f / 155925.f * z2 * z2 * z1;
-    c6 = 21844.f / 6081075.f * z2 * z2 * z2;
+    c2 = 2.f / 15.f * z1 * z1;
+    c3 = -17.f / 315.f * z1 * z1 * z1;
+    constexpr float k2 = 2.8853900817779268f, k2lo = (float)(2.8853900817779268 - (double)k2);
+    k = k2 * inv;
+    klo = __builtin_fmaf(__builtin_fmaf(-k, cap, k2), inv, k2lo * inv);
   }
-  __device__ __forceinline__ float low(float v) const {
-    const float z = v * v;
-    return __builtin_fmaf(v * z, __builtin_fmaf(__builtin_fmaf(c3, z, c2), z, c1), v);
+  __device__ __forceinline__ float low(float v, float& d) const {
+    const float z = v * v, t = __builtin_fmaf(v * z, __builtin_fmaf(__builtin_fmaf(c3, z, c2), z, c1), v);
+    const float th = t * inv;
+    d = __builtin_fmaf(-th, th, 1.f);
+    return t;
   }
-  __device__ __forceinline__ float mid(float v) const {
-    const float z = v * v;
-    float p = __builtin_fmaf(c6, z, c5);
-    p = __builtin_fmaf(p, z, c4);
-    p = __builtin_fmaf(p, z, c3);
-    p = __builtin_fmaf(p, z, c2);
-    p = __builtin_fmaf(p, z, c1);
-    return __builtin_fmaf(v * z, p, v);
+  __device__ __forceinline__ float mid(float v, float& d) const {
+    const float z = v * v * z1;
+    float p = -443861162.f / 1856156927625.f;
+    p = __builtin_fmaf(p, z, 6404582.f / 10854718875.f);
+    p = __builtin_fmaf(p, z, -929569.f / 638512875.f);
+    p = __builtin_fmaf(p, z, 21844.f / 6081075.f);
+    p = __builtin_fmaf(p, z, -1382.f / 155925.f);
+    p = __builtin_fmaf(p, z, 62.f / 2835.f);
+    p = __builtin_fmaf(p, z, -17.f / 315.f);
+    p = __builtin_fmaf(p, z, 2.f / 15.f);
+    p = __builtin_fmaf(p, z, -1.f / 3.f);
+    const float t = __builtin_fmaf(v * z, p, v), th = t * inv;
+    // (1 - th^2, with what th's rounding left out)
+    d = __builtin_fmaf(-2.f * th * inv, __builtin_fmaf(-th, cap, t), __builtin_fmaf(-th, th, 1.f));
+    return t;
   }
-  __device__ __forceinline__ float any(float v) const {
-    const float av = fabsf(v);
-    const float e = __builtin_amdgcn_exp2f(av * (2.8853900817779268f * inv));  // 2 log2(e) |v| / cap
-    const float big = copysignf(cap * __builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(e + 1.f), 1.f), v);
-    return av < 0.45f * cap ? mid(v) : big;
+  __device__ __forceinline__ float high(float v, float& d) const {
+    float av = fabsf(v);
+    av = av > 40.f * cap ? 40.f * cap : av;  // (e^80 is finite; NaN stays)
+    const float y = av * k, yl = __builtin_fmaf(av, klo, __builtin_fmaf(av, k, -y));
+    float e = __builtin_amdgcn_exp2f(y);
+    e = __builtin_fmaf(e * 0.69314718f, yl, e);
+    const float r = __builtin_amdgcn_rcpf(e + 1.f);
+    d = __builtin_fmaf(-4.f * r, r, 4.f * r);
+    return copysignf(__builtin_fmaf(-2.f * cap, r, cap), v);
   }
-  // f(value) over a lane's values of one column; ma = max |value| of the lane
+  __device__ __forceinline__ float any(float v, float& d) const {
+    float dm, dh;
+    const float m = mid(v, dm), h = high(v, dh);
+    const bool series = fabsf(v) < 0.6f * cap;
+    d = series ? dm : dh;
+    return series ? m : h;
+  }
+  // f(value, derivative) over a lane's values of one column; ma = max |value| of the lane
   template <typename F>
   __device__ __forceinline__ void over(float ma, F f) const {
-    if (__all(ma < cap * (1.f / 6.f))) f([this](float v) { return low(v); });
-    else if (__all(ma < 0.45f * cap)) f([this](float v) { return mid(v); });
-    else f([this](float v) { return any(v); });
+    if (__all(ma < cap * (1.f / 6.f))) f([this](float v, float& d) { return low(v, d); });
+    else if (__all(ma < 0.6f * cap)) f([this](float v, float& d) { return mid(v, d); });
+    else f([this](float v, float& d) { return any(v, d); });
   }
 };
 
@@ -317,8 +339,9 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[TM][TN], const GemmArgs
 #pragma unroll
           for (int r = 0; r < 16; r++) ma = fmaxf(ma, fabsf(acc[i][j][r]));
           sc.over(ma, [&](auto f) {
+            float d;
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r]);
+            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r], d);
           });
         }
     }
@@ -539,10 +562,11 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[TM][TN], const GemmArgs
           }
         scale = 1.f;
         Softcap(e.cap).over(ma, [&](auto f) {
+          float d;
 #pragma unroll
           for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r]);
+            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r], d);
         });
       }
 #pragma unroll
@@ -597,34 +621,26 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[TM][TN], const GemmArgs
       // per register one compare against a constant each
       const int tsel = e.targets[n] - ROW(0, 0), vend = e.vocab - ROW(0, 0);
       const float lsel = e.lse[n] * kLog2e, cs = e.colscale[n];
-      if (e.softcap) {
-        float ma = 0.f;
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-          for (int r = 0; r < 16; r++) ma = fmaxf(ma, fabsf(acc[i][j][r]));
-        Softcap(e.cap).over(ma, [&](auto f) {
-#pragma unroll
-          for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r]);
-        });
-      }
-      const float icap = 1.f / e.cap;
 #pragma unroll
       for (int i = 0; i < TM; i++) {
         half_t hv[16];
+        float dsc[16];
+#pragma unroll
+        for (int r = 0; r < 16; r++) dsc[r] = 1.f;
+        if (e.softcap) {
+          float ma = 0.f;
+#pragma unroll
+          for (int r = 0; r < 16; r++) ma = fmaxf(ma, fabsf(acc[i][j][r]));
+          Softcap(e.cap).over(ma, [&](auto f) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = f(acc[i][j][r], dsc[r]);
+          });
+        }
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const int mo = 32 * i + 8 * (r >> 2) + (r & 3);
-          const float v = acc[i][j][r];
-          float dsc = 1.f;
-          if (e.softcap) {
-            const float th = v * icap;
-            dsc = __builtin_fmaf(-th, th, 1.f);
-          }
-          float d = __builtin_amdgcn_exp2f(__builtin_fmaf(v, kLog2e, -lsel)) - (mo == tsel ? 1.f : 0.f);
-          d = mo < vend ? d * cs * dsc : 0.f;
+          float d = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[i][j][r], kLog2e, -lsel)) - (mo == tsel ? 1.f : 0.f);
+          d = mo < vend ? d * cs * dsc[r] : 0.f;
           hv[r] = (half_t)d;
           if (C) C[(size_t)ROW(i, r) * e.ldc + n] = hv[r];
         }
