@@ -205,18 +205,30 @@ struct Softcap {
     d = __builtin_fmaf(-4.f * r, r, 4.f * r);
     return copysignf(__builtin_fmaf(-2.f * cap, r, cap), v);
   }
+  // the value's own form, whatever the wave's other lanes hold; a form that no
+  // lane of the wave needs is skipped
   __device__ __forceinline__ float any(float v, float& d) const {
-    float dm, dh;
-    const float m = mid(v, dm), h = high(v, dh);
-    const bool series = fabsf(v) < 0.6f * cap;
-    d = series ? dm : dh;
-    return series ? m : h;
+    float t = low(v, d);
+    const bool in_low = fabsf(v) < cap * (1.f / 6.f), in_mid = fabsf(v) < 0.6f * cap;  // (false for NaN)
+    if (__any(!in_low)) {
+      float dm;
+      const float m = mid(v, dm);
+      t = in_low ? t : m;
+      d = in_low ? d : dm;
+    }
+    if (__any(!in_mid)) {
+      float dh;
+      const float h = high(v, dh);
+      t = in_mid ? t : h;
+      d = in_mid ? d : dh;
+    }
+    return t;
   }
-  // f(value, derivative) over a lane's values of one column; ma = max |value| of the lane
+  // f(value, derivative) over a lane's values of one column; ma = max |value|
+  // of the lane: one vote spares the votes on each value where all are low
   template <typename F>
   __device__ __forceinline__ void over(float ma, F f) const {
     if (__all(ma < cap * (1.f / 6.f))) f([this](float v, float& d) { return low(v, d); });
-    else if (__all(ma < 0.6f * cap)) f([this](float v, float& d) { return mid(v, d); });
     else f([this](float v, float& d) { return any(v, d); });
   }
 };

@@ -1,6 +1,7 @@
 """The softcap of the classifier epilogues over the magnitudes at which its form
 changes (cap / 6, 0.6 cap) and beyond, for logits, cross-entropy partials and
-the derivative in dlogits, against float64 tanh of the same fp32-exact logits.
+the derivative in dlogits, against float64 tanh of the same fp32-exact logits;
+and that a value's form is its own.
 
 A is diagonal and B selects one of its rows, so each logit is one exact product."""
 import ctypes as C
@@ -97,3 +98,32 @@ def test_softcap_derivative_does_not_cancel():
     assert normal[np.abs(v) > 100].any()
     err = np.abs(dl.astype(np.float64) - ref)[normal] / ref[normal]
     assert err.max() <= 2.0 ** -11 + 4e-6, err.max()
+
+
+@pytest.mark.parametrize("T", [512, 8192])
+def test_a_tokens_loss_does_not_depend_on_its_neighbours(T):
+    """The same tokens beside others whose logits are as small or far into the
+    cap: bit-identical log-sum-exps (128x128 and 256x256 tiles)."""
+    torch = pytest.importorskip("torch")
+    lib = _lib.load()
+    V, D, seq = 8192, 256, 64
+    r = np.random.default_rng(T)
+    xn = r.standard_normal((T, D)).astype(np.float16)
+    embed = (r.standard_normal((V, D)) * 0.02).astype(np.float16)
+    embed[:, :3] *= np.float16(4)  # a few logits past cap / 6 among the rest
+    tg = r.integers(0, V, T).astype(np.uint16)
+    beside = np.arange(T) % 7 == 3
+    dev = lambda a: torch.from_numpy(a.view(np.int16).copy()).cuda()
+    ptr = lambda t: C.c_void_p(t.data_ptr())
+    lses = []
+    for scale in (1.0, 4.0, 20.0):
+        x = xn.copy()
+        x[beside] *= np.float16(scale)
+        x_d, e_d, t_d = dev(x), dev(embed), dev(tg)
+        loss, lse = torch.zeros(T // seq, device="cuda"), torch.zeros(T, device="cuda")
+        assert lib.ane_head_loss(ptr(x_d), ptr(e_d), ptr(t_d), T, D, V, seq, 1, ptr(loss), ptr(lse),
+                                 C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0, lib.ane_op_last_error()
+        lses.append(lse.cpu().numpy())
+    assert (lses[0][beside] != lses[2][beside]).all()
+    for other in lses[1:]:
+        np.testing.assert_array_equal(other[~beside], lses[0][~beside])
