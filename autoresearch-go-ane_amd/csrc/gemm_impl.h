@@ -592,16 +592,19 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[TM][TN], const GemmArgs
           for (int r = 0; r < 16; r++) tv = (32 * i + 8 * (r >> 2) + (r & 3)) == tsel ? acc[i][j][r] : tv;
         tv *= scale;
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * scale;
-      // sum exp(v - max) as exp2(v log2e - max log2e): one FMA per value
+      // sum exp(v - max) as exp2(v log2e - max log2e): one FMA per value.  What
+      // the roundings of the scaled maximum and of the exponents' factor and
+      // offset come to at the maximum (3 2^-24 of it) is taken out of the sum.
       constexpr float kLog2e = 1.4426950408889634f;
-      const float mxl = mx * kLog2e, fac = scale * kLog2e;
+      const float mr = fmaxf(mx, __shfl_xor(mx, 32, 64)), fac = scale * kLog2e, mxl = mr * fac;
+      mx = mr * scale;
+      const float off = __builtin_fmaf(__builtin_fmaf(mr, scale, -mx), kLog2e, -__builtin_fmaf(mr, fac, -mxl));
       float s = 0.f;
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) s += __builtin_amdgcn_exp2f(__builtin_fmaf(acc[i][j][r], fac, -mxl));
-      s += __shfl_xor(s, 32, 64);
+      s = (s + __shfl_xor(s, 32, 64)) * __builtin_amdgcn_exp2f(off);
       if (hit) e.tgt_logit[n] = tv;  // exactly one lane of the grid holds (tg, n)
       if (lane < 32) red[wm * BN + nl] = make_float2(mx, s);
     }

@@ -17,7 +17,7 @@ import pytest
 
 import ane
 import oracle
-from ane import _lib
+from ane import _lib, hsaco
 
 pytestmark = pytest.mark.gpu
 
@@ -123,3 +123,41 @@ def test_forward_with_and_without_norm_launches(monkeypatch):
     print("per-sequence loss deferred", per["1"], "launches", per["0"], "oracle", per_ref)
     np.testing.assert_allclose(per["1"], per["0"], atol=5e-4)
     np.testing.assert_allclose(per["1"], per_ref, atol=1e-3)
+
+
+def test_classifier_sum_with_the_norm_folded_in():
+    """Log-sum-exps of logits near 500 from the exported classifier kernel,
+    1 / rms in the exponentials' factor.  Each logit is one exact fp16 value
+    times the column's 1 / rms.  Bound: the 256 exponentials and their sum
+    (2^-24 each step; the terms that matter have arguments below 8, off by
+    2^-21).  The maximum's and the factor's roundings, 3 2^-24 of 500, are not
+    in it."""
+    hip = hsaco.Hip()
+    co = hsaco.CodeObjects(hip)
+    V = T = D = 256
+    r = np.random.default_rng(17)
+    v = (500 + 0.25 * r.integers(-32, 33, V)).astype(np.float16)
+    a = np.zeros((V, D), np.float16)
+    a[np.arange(V), np.arange(V)] = v
+    part = (r.random((1, T)) * 8 + 0.1).astype(np.float32)
+    rr = np.float32(1) / np.sqrt(part[0] / np.float32(4) + np.float32(1e-5))  # rr_dim 4
+    tgt = r.integers(0, V, T).astype(np.uint16)
+    bufs = [hip.upload(x) for x in (a, np.ones((T, D), np.float16), tgt, part, np.zeros((T, 2), np.float32),
+                                    np.zeros(T, np.float32))]
+    try:
+        g = hsaco._gemm(V, T, D, bufs[0], D, bufs[1], D)
+        e = hsaco.AneEpiParams(targets=bufs[2], partial=bufs[4], tgt_logit=bufs[5], softcap=0, cap=15.0, vocab=V,
+                               scale=1.0, alpha=1.0, rr_part=bufs[3], rr_ld=T, rr_nparts=1, rr_dim=4)
+        co.launch("gemm", "ane_k_gemm_ce_rr", (1,), 512, g, e)
+        hip.check(hip.lib.hipDeviceSynchronize(), "hipDeviceSynchronize")
+        pm, ps = hip.download(bufs[4], (T, 2), np.float32).astype(np.float64).T
+        tl = hip.download(bufs[5], (T,), np.float32)
+    finally:
+        for b in bufs:
+            hip.lib.hipFree(C.c_void_p(b))
+        co.close()
+    x = v.astype(np.float64)[:, None] * rr.astype(np.float64)
+    m = x.max(0)
+    lse = m + np.log(np.exp(x - m).sum(0))
+    np.testing.assert_array_equal(tl, (v[tgt].astype(np.float32) * rr))
+    np.testing.assert_allclose(pm + np.log(ps), lse, rtol=0, atol=4e-6)
