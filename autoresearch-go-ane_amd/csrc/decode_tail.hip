@@ -251,7 +251,7 @@ __device__ __forceinline__ int x_index(int cg, int D, int nb) {
 // pair of x[:, cg], loaded before the GEMM) += acc and is stored; ssq[cg][t] = sum
 // over the group's 32 columns of the new x^2; xg = fp16(x * gain) fragments
 // for the consumer.  Rows below nb.
-__device__ void resid_epilogue(float (*red)[64][32], float2 xv, int cg, float* x, int D, float* ssq, half_t* xg,
+__device__ __forceinline__ void resid_epilogue(float (*red)[64][32], float2 xv, int cg, float* x, int D, float* ssq, half_t* xg,
                                const float* gain, int nb) {
   const int row = threadIdx.x >> 4, c = cg * 32 + (threadIdx.x & 15) * 2;
   if (row >= nb) return;
