@@ -56,7 +56,8 @@ struct AttnBwdArgs {
 
 // seq <= 256 (the whole sequence is staged in LDS twice).
 hipError_t attention_bwd(const AttnBwdArgs& a, hipStream_t stream);
-// The same for few (sequence, head) pairs, by attention_bwd's rule.
+// The same for few (sequence, head) pairs, by attention_bwd's rule; each block
+// forms the delta of its rows, the buffer is not used.
 hipError_t attention_bwd_few(const AttnBwdArgs& a, hipStream_t stream);
 
 }  // namespace ane

@@ -542,7 +542,9 @@ hipError_t attention_fwd(const AttnArgs& a, hipStream_t stream) {
   // 24 14.5 / 10.7, 36 14.5 / 15.0; S = 128 48 heads 11.6 / 9.0; S = 512 12
   // heads 25.3 / 14.3, 24 24.8 / 20.4, 36 25.1 / 27.8; S = 320 48 heads 20.9 /
   // 15.1, 72 20.4 / 22.7.
-  if ((long)a.nseq * a.NH * (a.S / 32) <= (a.S > 256 ? 512 : 256)) return attention_fwd_few(a, stream);
+  // (Split operands that are also kept, which no caller asks for, have no few-heads form.)
+  if ((long)a.nseq * a.NH * (a.S / 32) <= (a.S > 256 ? 512 : 256) && !(a.hilo && a.qkvt_lo))
+    return attention_fwd_few(a, stream);
   const int npairs = a.S / 64;
   const int nw = npairs < 4 ? npairs : 4;  // q-block pairs per block
   dim3 grid((npairs + nw - 1) / nw, a.NH, a.nseq);

@@ -411,7 +411,6 @@ __global__ __launch_bounds__(64 * NWV) void attn_bwd_few_kernel(AttnBwdArgs a) {
     if constexpr (HILO) qlo = ld_frag(lob + (size_t)q * 2 * D, g);
     const float lse2 = a.lse[t * NH + h] * kLog2e;
     const float dd = frag_dot(df, of);
-    if (wave == 0 && g == 0) a.delta[t * NH + h] = dd;
     floatx16 dq0, dq1;
 #pragma unroll
     for (int r = 0; r < 16; r++) dq0[r] = dq1[r] = 0.f;
@@ -553,8 +552,8 @@ hipError_t attention_fwd_few(const AttnArgs& a, hipStream_t stream) {
   const dim3 grid(a.S / 32, a.NH, a.nseq);
 #define FEW(HILO_, LO_) hipLaunchKernelGGL((attn_fwd_few_kernel<HILO_, LO_>), grid, dim3(64 * NWV), 0, stream, a)
   if (a.hilo) {
-    if (a.qkvt_lo) FEW(true, true);
-    else FEW(true, false);
+    if (a.qkvt_lo) return hipErrorInvalidValue;  // (attention_fwd's rule leaves it to the other kernels)
+    FEW(true, false);
   } else if (a.qkvt_lo) {
     FEW(false, true);
   } else {
