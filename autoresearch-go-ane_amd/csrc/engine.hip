@@ -1162,27 +1162,33 @@ done:
 //   STORE_H, RELU2: C fp16 [M, N];  RELU2: C2 fp16 [M, N] (pre-activation)
 //   SWIGLU: C fp16 [M, N/2] over 32-column interleaved W1|W3, C2 fp16 [M, N]
 //   STORE_F, LOGITS (softcap = 15 when seq < 0), RESID, SMEAR: C fp32 [M, N]
+//   STORE_F with R: C += (R in C before)
 //   RESID: R fp32 [M, N] (C = alpha R + acc + beta X0; X0 optional; C2 fp32
-//          copy optional);  SMEAR: X0 fp32 [M, N], rows t with t % seq == 0
-//          have no predecessor, C2 fp32 gate
+//          copy optional; seq != 0: alpha and beta read from device memory);
+//   SMEAR: X0 fp32 [M, N], rows t with t % seq == 0 have no predecessor, C2
+//          fp32 gate
+//   SWIGLU_BWD: C2 in, C out fp16 [M, 2 N], h1|h3 and dh1|dh3 in 32-column
+//          interleave;  RELU2_BWD: C2 in, C out fp16 [M, N]
 // C2 / X0 / R may be NULL where optional.
 extern "C" int ane_debug_gemm_epi(int epi, int M, int N, int K, const uint16_t* A, const uint16_t* B, void* C,
                                   void* C2, const float* X0, const float* R, float alpha, float beta, int seq, int bm,
                                   int bn, int nw) {
   const bool f32 = epi == EPI_STORE_F || epi == EPI_LOGITS || epi == EPI_RESID || epi == EPI_SMEAR;
-  if (!f32 && epi != EPI_STORE_H && epi != EPI_RELU2 && epi != EPI_SWIGLU) {
+  const bool bwd = epi == EPI_SWIGLU_BWD || epi == EPI_RELU2_BWD;
+  if (!f32 && !bwd && epi != EPI_STORE_H && epi != EPI_RELU2 && epi != EPI_SWIGLU) {
     g_debug_err = "storiesane debug: unsupported epilogue";
     return ANE_ERR_ARG;
   }
-  if ((epi == EPI_RESID && !R) || (epi == EPI_SMEAR && (!X0 || seq <= 0))) {
+  if ((epi == EPI_RESID && !R) || (epi == EPI_SMEAR && (!X0 || seq <= 0)) || (bwd && !C2)) {
     g_debug_err = "storiesane debug: missing epilogue operand";
     return ANE_ERR_ARG;
   }
   int rc = ANE_OK;
-  void *dA = nullptr, *dB = nullptr, *dC = nullptr, *dC2 = nullptr, *dX0 = nullptr, *dR = nullptr;
+  void *dA = nullptr, *dB = nullptr, *dC = nullptr, *dC2 = nullptr, *dX0 = nullptr, *dR = nullptr, *dS = nullptr;
   const size_t MN = (size_t)M * N;
-  const size_t cbytes = epi == EPI_SWIGLU ? MN : (f32 ? MN * 4 : MN * 2);
-  const size_t c2bytes = (epi == EPI_RESID || epi == EPI_SMEAR) ? MN * 4 : MN * 2;
+  const size_t cbytes = epi == EPI_SWIGLU ? MN : (f32 || epi == EPI_SWIGLU_BWD ? MN * 4 : MN * 2);
+  const size_t c2bytes = (epi == EPI_RESID || epi == EPI_SMEAR || epi == EPI_SWIGLU_BWD) ? MN * 4 : MN * 2;
+  const float ab[2] = {alpha, beta};
   GemmArgs g;
   EpiParams p;
   DBGCHK(hipMalloc(&dA, (size_t)M * K * 2));
@@ -1191,6 +1197,17 @@ extern "C" int ane_debug_gemm_epi(int epi, int M, int N, int K, const uint16_t* 
   DBGCHK(hipMemcpy(dA, A, (size_t)M * K * 2, hipMemcpyHostToDevice));
   DBGCHK(hipMemcpy(dB, B, (size_t)N * K * 2, hipMemcpyHostToDevice));
   if (C2) DBGCHK(hipMalloc(&dC2, c2bytes));
+  if (bwd) DBGCHK(hipMemcpy(dC2, C2, c2bytes, hipMemcpyHostToDevice));
+  if (epi == EPI_STORE_F && R) {
+    DBGCHK(hipMemcpy(dC, R, cbytes, hipMemcpyHostToDevice));
+    p.accumulate = 1;
+  }
+  if (epi == EPI_RESID && seq) {
+    DBGCHK(hipMalloc(&dS, sizeof ab));
+    DBGCHK(hipMemcpy(dS, ab, sizeof ab, hipMemcpyHostToDevice));
+    p.alpha_ptr = (const float*)dS; p.beta_ptr = (const float*)dS + 1;
+    alpha = beta = 0.f;
+  }
   if (X0) {
     DBGCHK(hipMalloc(&dX0, MN * 4));
     DBGCHK(hipMemcpy(dX0, X0, MN * 4, hipMemcpyHostToDevice));
@@ -1201,8 +1218,8 @@ extern "C" int ane_debug_gemm_epi(int epi, int M, int N, int K, const uint16_t* 
   }
   g.A = (const half_t*)dA; g.B = (const half_t*)dB;
   g.lda = K; g.ldb = K; g.M = M; g.N = N; g.K = K; g.a_t = false; g.b_t = false;
-  p.C = dC; p.ldc = epi == EPI_SWIGLU ? N / 2 : N;
-  p.C2 = dC2; p.ldc2 = N;
+  p.C = dC; p.ldc = epi == EPI_SWIGLU ? N / 2 : epi == EPI_SWIGLU_BWD ? 2 * N : N;
+  p.C2 = dC2; p.ldc2 = epi == EPI_SWIGLU_BWD ? 2 * N : N;
   p.X0 = (const float*)dX0; p.R = (const float*)dR;
   p.alpha = alpha; p.beta = beta; p.seq = seq;
   if (epi == EPI_LOGITS && seq < 0) { p.softcap = 1; p.cap = 15.f; }
@@ -1211,12 +1228,14 @@ extern "C" int ane_debug_gemm_epi(int epi, int M, int N, int K, const uint16_t* 
   DBGCHK(hipMemcpy(C, dC, cbytes, hipMemcpyDeviceToHost));
   if (C2) DBGCHK(hipMemcpy(C2, dC2, c2bytes, hipMemcpyDeviceToHost));
 done:
-  for (void* q : {dA, dB, dC, dC2, dX0, dR})
+  for (void* q : {dA, dB, dC, dC2, dX0, dR, dS})
     if (q) (void)hipFree(q);
   return rc;
 }
 
-// The deferred-RMSNorm epilogues on one forced tile (host buffers).
+// The deferred-RMSNorm epilogues (host buffers) on one forced tile, or, bm =
+// bn = 0, where gemm_run's thin form takes the shape (ssq per 64 columns;
+// nw < 0: with a gain that is not 16-byte aligned, which that form refuses).
 // epi 13 (EPI_RESID_NORM): X [M, N] fp32 in/out (X += acc), C [M, N] fp16 =
 // X * gain[col], ssq [N / bn][M] = per-row sums of X^2 over each block's bn
 // columns.  epi 14 (EPI_STORE_H_RR): C [M, N] fp16 = acc * rr[row]; epi 15
@@ -1226,7 +1245,10 @@ done:
 extern "C" int ane_debug_gemm_norm(int epi, int M, int N, int K, const uint16_t* A, const uint16_t* B, float* X,
                                    uint16_t* C, const float* gain, float* ssq, const float* rr_part, int nparts,
                                    int rr_dim, int bm, int bn, int nw) {
-  if ((epi != EPI_RESID_NORM && epi != EPI_STORE_H_RR && epi != EPI_SWIGLU_RR) || bm <= 0 || bn <= 0 ||
+  const bool thin = bm == 0 && bn == 0 && gemm_pick_thin(M, N, K, epi).bm;
+  const bool off = thin && nw < 0;
+  if (thin) nw = 0;
+  if ((epi != EPI_RESID_NORM && epi != EPI_STORE_H_RR && epi != EPI_SWIGLU_RR) || (!thin && (bm <= 0 || bn <= 0)) ||
       (epi == EPI_RESID_NORM && (!X || !gain || !ssq)) || (epi != EPI_RESID_NORM && (!rr_part || nparts < 1))) {
     g_debug_err = "storiesane debug: unsupported deferred-norm epilogue or missing operand";
     return ANE_ERR_ARG;
@@ -1235,7 +1257,7 @@ extern "C" int ane_debug_gemm_norm(int epi, int M, int N, int K, const uint16_t*
   void *dA = nullptr, *dB = nullptr, *dC = nullptr, *dX = nullptr, *dG = nullptr, *dS = nullptr, *dP = nullptr;
   const size_t MN = (size_t)M * N;
   const size_t cbytes = epi == EPI_SWIGLU_RR ? MN : MN * 2;
-  const size_t sbytes = (size_t)(N / bn) * M * 4;
+  const size_t sbytes = (size_t)(N / (thin ? 64 : bn)) * M * 4;
   GemmArgs g;
   EpiParams p;
   DBGCHK(hipMalloc(&dA, (size_t)M * K * 2));
@@ -1245,11 +1267,11 @@ extern "C" int ane_debug_gemm_norm(int epi, int M, int N, int K, const uint16_t*
   DBGCHK(hipMemcpy(dB, B, (size_t)N * K * 2, hipMemcpyHostToDevice));
   if (epi == EPI_RESID_NORM) {
     DBGCHK(hipMalloc(&dX, MN * 4));
-    DBGCHK(hipMalloc(&dG, (size_t)N * 4));
+    DBGCHK(hipMalloc(&dG, (size_t)N * 4 + 4));
     DBGCHK(hipMalloc(&dS, sbytes));
     DBGCHK(hipMemcpy(dX, X, MN * 4, hipMemcpyHostToDevice));
-    DBGCHK(hipMemcpy(dG, gain, (size_t)N * 4, hipMemcpyHostToDevice));
-    p.C = dX; p.ldc = N; p.R = (const float*)dX; p.C2 = dC; p.ldc2 = N; p.gain = (const float*)dG;
+    DBGCHK(hipMemcpy((float*)dG + off, gain, (size_t)N * 4, hipMemcpyHostToDevice));
+    p.C = dX; p.ldc = N; p.R = (const float*)dX; p.C2 = dC; p.ldc2 = N; p.gain = (const float*)dG + off;
     p.ssq_part = (float*)dS; p.ssq_ld = M;
   } else {
     DBGCHK(hipMalloc(&dP, (size_t)nparts * M * 4));

@@ -252,16 +252,21 @@ int ane_sync(ane_engine *e);
  * Messages: ane_debug_last_error(). */
 int ane_debug_gemm(int a_t, int b_t, int epi, int M, int N, int K, const uint16_t *A, const uint16_t *B,
                    void *C, int bm, int bn, int nw, int ns, int splits);
-/* One K-major GEMM (A [M, K], B [N, K]) with a fused forward epilogue on host
- * buffers (epi: 0 fp16 store, 1 fp32 store, 2 logits (softcap 15 when
- * seq < 0), 3 residual C = alpha R + acc + beta X0 (+ copy to C2), 4 SwiGLU
+/* One K-major GEMM (A [M, K], B [N, K]) with a fused epilogue on host
+ * buffers (epi: 0 fp16 store, 1 fp32 store (added to R when given), 2 logits
+ * (softcap 15 when seq < 0), 3 residual C = alpha R + acc + beta X0 (+ copy to
+ * C2; seq != 0: alpha and beta read from device memory), 4 SwiGLU
  * over 32-column interleaved W1|W3 (C fp16 [M, N/2], C2 fp16 h1|h3), 5
- * relu^2 (C2 = pre-activation), 6 smear (X0, seq; C2 = gate)).  Optional
- * operands may be NULL. */
+ * relu^2 (C2 = pre-activation), 6 smear (X0, seq; C2 = gate), 10 SwiGLU
+ * backward (C2 fp16 h1|h3 in, C fp16 dh1|dh3, both [M, 2N]), 11 relu^2
+ * backward (C2 fp16 pre-activation in, C fp16)).  Optional operands may be
+ * NULL. */
 int ane_debug_gemm_epi(int epi, int M, int N, int K, const uint16_t *A, const uint16_t *B, void *C, void *C2,
                        const float *X0, const float *R, float alpha, float beta, int seq, int bm, int bn, int nw);
 /* The deferred-RMSNorm epilogues of the llama2 eval forward on one forced
- * tile (bm x bn, nw waves): epi 13: X [M, N] fp32 in/out (X += A B^T),
+ * tile (bm x bn, nw waves; bm = bn = 0: the kernel for small outputs, where the
+ * shape is one of its own, ssq per 64 columns; nw < 0: with an unaligned gain,
+ * for which the dispatch takes another kernel): epi 13: X [M, N] fp32 in/out (X += A B^T),
  * C [M, N] fp16 = X * gain[col], ssq [N/bn][M] = per-row sums of X^2 over
  * each block's bn columns; epi 14: C [M, N] fp16 = (A B^T) * rr[row]; epi 15:
  * C [M, N/2] fp16 = SwiGLU over 32-column interleaved W1|W3 of (A B^T) *

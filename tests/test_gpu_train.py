@@ -62,8 +62,9 @@ def test_tiny_grads_match_oracle(arch, mode):
 @pytest.mark.parametrize("seq", [128, 192])
 @pytest.mark.parametrize("arch,mode", [("llama2", "true"), ("nanochat", "compat")])
 def test_tiny_grads_at_other_sequence_lengths(arch, mode, seq):
-    """Sequences of 2 and 3 pairs of 32-query blocks: the attention backward
-    then runs 2 and 3 waves per block (4 at seq 256, 1 at seq 64)."""
+    """Sequences of 4 and 6 32-query blocks, few enough heads for a block of
+    the attention backward per 32 rows (test_gpu_attention_few.py has the
+    kernels that run 2 and 3 waves per block at these lengths)."""
     cfg = ane.tiny(arch, layers=2, grad_mode=mode, seq=seq)
     p = ane.init_params(cfg, seed=23, std=0.08)
     tok, tgt = ane.make_tokens(cfg, 2, seed=24)
