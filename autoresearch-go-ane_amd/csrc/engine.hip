@@ -780,7 +780,11 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
       EpiParams p;
       p.C = A.qkv; p.ldc = 3 * D;
       if (fused) rr(p, nparts);
-      // its weights were streamed by the previous layer's W2 GEMM (layer 0: by the embedding)
+      // its weights were streamed by the previous layer's W2 GEMM (layer 0: by
+      // the embedding), unless one of the two is thin.  Where only W2's is, a
+      // prefetch launch instead costs more than it gives: evaluation, us,
+      // without / with, 4 windows of 256 793 / 815, 6 915 / 939, 8 1086 / 1090,
+      // 10 1189 / 1208, 5 of 448 1250 / 1266
       HIPCHK(op, eng_gemm(e, 0, A.xn, D, false, s.wqkv, D, false, T, 3 * D, D, fused ? EPI_STORE_H_RR : EPI_STORE_H,
                           p));
     }
@@ -853,7 +857,8 @@ int forward_body(ane_engine* e, int nseq, int train, bool defer_norm) {
         p.ssq_part = e->ssq_part; p.ssq_ld = T;
         // streams the next layer's Wq|Wk|Wv (the classifier's come by a prefetch launch)
         (void)res_tile(H);
-        const void* pf2 = e->gemm_selfpf && qkv_ahead && l + 1 < L ? (const void*)e->ls[l + 1].wqkv : nullptr;
+        const bool ahead2 = e->gemm_selfpf && res_bn && qkv_ahead && l + 1 < L;  // (thin GEMMs stream nothing)
+        const void* pf2 = ahead2 ? (const void*)e->ls[l + 1].wqkv : nullptr;
         HIPCHK(op, eng_gemm(e, 3, A.gate, H, false, s.w2, H, false, T, D, H, EPI_RESID_NORM, p, res_bm, res_bn, false,
                             pf2, (size_t)3 * D * D * sizeof(half_t)));
         nparts = D / res_cols;

@@ -260,8 +260,13 @@ int backward_body(ane_engine* e, int nseq, bool async) {
   // meet each B panel at once and a 64x64-tile GEMM pays ~10 us (W1|W3 dX
   // and dW at B16).  A prefetch issued a few kernels earlier does not help:
   // the data in between evicts it.
-  // Few tokens: the dX GEMMs run as gemm_thin_kernel, which requests its
-  // operands whole, and the saved activations are still in the caches.
+  // None while the W1|W3 dX GEMM runs as gemm_thin_kernel (768 wide: up to
+  // about 2700 tokens): that kernel requests its operands whole, and what the
+  // other GEMMs gain is what the launches cost.  A step of 12 layers of 768, ms,
+  // without / with prefetch launches (of what thin GEMMs do not read): 1
+  // window of 256 1.60 / 1.80, 2 1.93 / 1.97, 4 2.72 / 2.66, 5 2.99 / 2.95, 6
+  // 3.27 / 3.29, 8 3.90 / 3.86, 10 4.27 / 4.24; nanochat 2 2.13 / 2.12, 5 3.29 /
+  // 3.28, 8 4.30 / 4.33.
   const bool bwd_ahead = e->bwd_prefetch && !gemm_pick_thin(T, D, KH, EPI_STORE_F).bm;
   auto prefetch = [&](hipStream_t s, std::initializer_list<std::pair<const void*, size_t>> regions) -> hipError_t {
     if (!bwd_ahead) return hipSuccess;
