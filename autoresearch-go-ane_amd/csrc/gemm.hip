@@ -96,7 +96,11 @@ void gemm_pick_split(int M, int N, int K, int epi, size_t ws_cap, int* pbm, int*
   //  (c) long K with fewer than 512 blocks of the default tile (dW of
   //      Wq|Wk|Wv, Wo, W2): the largest tile and fewest splits reaching 384
   //      blocks with >= 512 k per split (Wo: 18.5 us vs 32.3; W2 28.0 vs
-  //      34.6; QKV 29.3 vs 36.5).
+  //      34.6; QKV 29.3 vs 36.5), or else the most blocks there are (K with
+  //      few divisors, narrow models: unsplit, the weight gradients outlast
+  //      the main stream's kernels, and what those gain slows them further.
+  //      A nanochat step of 4 layers of 256, unsplit / so, us: 3072 tokens 971
+  //      / 770, 4032 1285 / 929, 5888 1821 / 1254).
   // Otherwise the plain heuristic, one pass.
   int bm = 0, bn = 0;
   gemm_pick_tile(M, N, K, epi, &bm, &bn);
@@ -130,16 +134,16 @@ void gemm_pick_split(int M, int N, int K, int epi, size_t ws_cap, int* pbm, int*
   }
   if (K < 2048 || (long)(M / bm) * (N / bn) >= 512) return;
   static const int cand[][2] = {{128, 128}, {64, 128}, {128, 64}, {64, 64}};
+  long most = (long)(M / bm) * (N / bn);
   for (const auto& c : cand) {
     if (M % c[0] || N % c[1]) continue;
     const long t = (long)(M / c[0]) * (N / c[1]);
     for (int sp = 2; sp <= 16; sp++) {
       if (K / sp < 512) break;
-      if (!fits(sp)) continue;
-      if (t * sp >= 384) {
-        *pbm = c[0]; *pbn = c[1]; *psplits = sp;
-        return;
-      }
+      if (!fits(sp) || (t * sp < 384 && t * sp <= most)) continue;
+      most = t * sp;
+      *pbm = c[0]; *pbn = c[1]; *psplits = sp;
+      if (most >= 384) return;
     }
   }
 }
