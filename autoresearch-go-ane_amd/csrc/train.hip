@@ -267,7 +267,17 @@ int backward_body(ane_engine* e, int nseq, bool async) {
   // window of 256 1.60 / 1.80, 2 1.93 / 1.97, 4 2.72 / 2.66, 5 2.99 / 2.95, 6
   // 3.27 / 3.29, 8 3.90 / 3.86, 10 4.27 / 4.24; nanochat 2 2.13 / 2.12, 5 3.29 /
   // 3.28, 8 4.30 / 4.33.
-  const bool bwd_ahead = e->bwd_prefetch && !gemm_pick_thin(T, D, KH, EPI_STORE_F).bm;
+  // Except where T has no divisor to split the weight gradients by, from 1.2 M
+  // activations on: those GEMMs then walk cold k-tiles one after another and
+  // end last.  A nanochat step of 4 layers, without / with, us: 5056 tokens x
+  // 256 1544 / 1452, 3776 x 512 1649 / 1588 (3776 x 256 1140 / 1171).
+  auto dw_unsplit = [&] {
+    int bm = 0, bn = 0, sp = 1;
+    gemm_pick_split(D, D, T, EPI_STORE_F, tb.splitk_cap, &bm, &bn, &sp);
+    return sp == 1;
+  };
+  const bool bwd_ahead = e->bwd_prefetch && (!gemm_pick_thin(T, D, KH, EPI_STORE_F).bm ||
+                                             ((long)T * D >= 1200 * 1024 && dw_unsplit()));
   auto prefetch = [&](hipStream_t s, std::initializer_list<std::pair<const void*, size_t>> regions) -> hipError_t {
     if (!bwd_ahead) return hipSuccess;
     PrefetchList pl;
