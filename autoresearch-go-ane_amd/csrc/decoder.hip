@@ -554,7 +554,7 @@ extern "C" int ane_decode_set_params(ane_decoder* d, const float* params, int64_
     DCHK(op, weight_to_frag(d->fw2 + (size_t)l * D * H, d->w2 + (size_t)l * D * H, D, H, st));
   }
   DCHK(op, weight_to_frag(d->fembed, d->embed_h, d->V, D, st));
-  DCHK(op, hc.finish());
+  DCHK(op, hc.finish(false));
   d->params_set = true;
   return ANE_OK;
 }

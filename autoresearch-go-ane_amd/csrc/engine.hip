@@ -626,7 +626,7 @@ extern "C" int ane_set_params(ane_engine* e, const float* params, int64_t n) {
   HIPCHK("set params", hc.up(e->P, params, (size_t)n * 4));
   int rc = refresh_shadows(e);
   if (rc) return rc;
-  HIPCHK("set params", hc.finish());
+  HIPCHK("set params", hc.finish(false));
   return ANE_OK;
 }
 

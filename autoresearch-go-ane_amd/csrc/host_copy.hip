@@ -306,7 +306,7 @@ hipError_t HostCopy::down(void* dst, const void* src, size_t n) {
   return hipSuccess;
 }
 
-hipError_t HostCopy::finish() {
+hipError_t HostCopy::finish(bool poll) {
   hipError_t h = hipSuccess;
   if (p_) {
     while (n_pending_ > 0) {
@@ -316,7 +316,7 @@ hipError_t HostCopy::finish() {
     for (HostPool::Slot& s : p_->slots_) drain(&s.left);
     drain(&p_->touched_);
   }
-  const hipError_t r = stream_wait(st_);
+  const hipError_t r = poll ? stream_wait(st_) : hipStreamSynchronize(st_);
   return h == hipSuccess ? r : h;
 }
 

@@ -412,7 +412,7 @@ extern "C" int ane_moe_set_params(ane_moe* m, const float* params, int64_t n) {
     MCHK(op, interleave_w13(m->w13 + (size_t)e * 2 * H * D, base, base + H * D, (int)H, (int)D, st));
     MCHK(op, f32_to_f16(m->w2 + (size_t)e * D * H, base + 2 * H * D, D * H, st));
   }
-  MCHK(op, hc.finish());
+  MCHK(op, hc.finish(false));
   m->params_set = true;
   return ANE_OK;
 }

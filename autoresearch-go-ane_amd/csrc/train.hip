@@ -884,7 +884,7 @@ extern "C" int ane_set_grads(ane_engine* e, const float* grads, int64_t n, uint3
   if (rc) return rc;
   HostCopy hc(&e->host_pool, e->device, e->stream);
   HIPCHK(op, hc.up(e->tr.G, grads, (size_t)n * 4));
-  HIPCHK(op, hc.finish());
+  HIPCHK(op, hc.finish(false));
   e->state.pending_steps = pending;
   return ANE_OK;
 }
@@ -919,7 +919,7 @@ extern "C" int ane_set_opt_state(ane_engine* e, const float* m, const float* v, 
   else HIPCHK(op, hipMemsetAsync(e->tr.M, 0, (size_t)n * 4, e->stream));
   if (v) HIPCHK(op, hc.up(e->tr.Vv, v, (size_t)n * 4));
   else HIPCHK(op, hipMemsetAsync(e->tr.Vv, 0, (size_t)n * 4, e->stream));
-  HIPCHK(op, hc.finish());
+  HIPCHK(op, hc.finish(false));
   return ANE_OK;
 }
 
