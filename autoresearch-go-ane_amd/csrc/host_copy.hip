@@ -191,6 +191,7 @@ bool HostCopy::take(const void* host, size_t n) {
     return false;
   }
   p_ = ref_->pool.get();
+  p_->next_ = 0;  // (the slots of small calls stay in the caches, and later ones are not paged in for them)
   return true;
 }
 
