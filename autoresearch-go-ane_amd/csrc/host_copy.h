@@ -33,8 +33,14 @@ class HostPool {
   static constexpr size_t kSlotBytes = (size_t)4 << 20;
   static constexpr size_t kTaskBytes = (size_t)256 << 10;  // one thread's piece of a slot
   static constexpr int kThreads = 6;
-  // below this a copy is left to hipMemcpyAsync: waking the threads costs more
-  static constexpr size_t kMinBytes = (size_t)256 << 10;
+  // Below this a copy is left to hipMemcpyAsync: waking the threads costs more
+  // (us a call, hipMemcpyAsync / pool, to the host 368 KB 25 / 45, 880 KB 46 /
+  // 56, 1.1 MB 73 / 62, 2.1 MB 133 / 87; from it 33 / 46, 52 / 56, 73 / 62, 102 /
+  // 82).  A call of many copies, or one that has the pool already, uses it
+  // from kMoreBytes on (one layer's forward with its ten taps, 512 wide, 128
+  // positions, 256 KB a copy: 465 / 398).
+  static constexpr size_t kMinBytes = (size_t)1 << 20;
+  static constexpr size_t kMoreBytes = (size_t)256 << 10;
   // what an object has to copy before a pool is made for it (one that is
   // there already is used at once): making it, 32 MB of pinned memory and the
   // threads, costs about what the pool saves on 8 MB.  Opening and closing a
@@ -103,7 +109,9 @@ struct HostPoolRef {
 class HostCopy {
  public:
   // ref: the calling object's, filled by the copy from which the pool pays
-  HostCopy(HostPoolRef* ref, int device, hipStream_t st) : ref_(ref), device_(device), st_(st) {}
+  // many: the call has eight copies or more
+  HostCopy(HostPoolRef* ref, int device, hipStream_t st, bool many = false)
+      : ref_(ref), device_(device), st_(st), min_(many ? HostPool::kMoreBytes : HostPool::kMinBytes) {}
   ~HostCopy();
   HostCopy(const HostCopy&) = delete;
   HostCopy& operator=(const HostCopy&) = delete;
@@ -124,6 +132,7 @@ class HostCopy {
   HostPoolRef* ref_;
   int device_;
   hipStream_t st_;
+  size_t min_;                                    // least copy for which the pool is taken
   HostPool* p_ = nullptr;                         // locked
   bool busy_ = false;                             // another thread has the pool, or there is none: not asked again
   int pending_[HostPool::kSlots];                 // slots queued to the host: n_pending_ from first_, oldest first

@@ -170,7 +170,7 @@ void HostPool::wake() {
 // ---- one call's copies ---------------------------------------------------------
 
 bool HostCopy::take(const void* host, size_t n) {
-  if (n < HostPool::kMinBytes || busy_) return false;
+  if (n < (p_ ? HostPool::kMoreBytes : min_) || busy_) return false;
   // memory the runtime already has pinned (or managed) is copied directly
   hipPointerAttribute_t at;
   memset(&at, 0, sizeof at);

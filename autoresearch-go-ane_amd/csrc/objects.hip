@@ -247,7 +247,7 @@ struct SeamBase {
 struct Copies {
   SeamBase* b;
   HostCopy hc;
-  explicit Copies(SeamBase* o) : b(o), hc(&o->pool, o->device, o->st) { b->copies = &hc; }
+  explicit Copies(SeamBase* o, bool many = false) : b(o), hc(&o->pool, o->device, o->st, many) { b->copies = &hc; }
   ~Copies() { b->copies = nullptr; }
 };
 
@@ -391,7 +391,7 @@ int layer_forward_call(ane_layer_fwd* f, float* out, const float* x, ane_layer_c
   const size_t DS = (size_t)D * S, HS = (size_t)H * S;
   hipStream_t st = f->st;
   SEAMCHK(op, f->enter());
-  Copies copies(f);
+  Copies copies(f, cache != nullptr);
   SEAMCHK(op, f->up(f->xcf, x, DS * 4));
   SEAMCHK(op, layer_forward_device(f));
   SEAMCHK(op, (xpose<float, float>(f->cf, f->y, S, D, D, S, st)));
@@ -600,7 +600,7 @@ extern "C" int ane_layer_backward_run_attention(ane_layer_bwd* lb, float* dx_nor
   const int D = lb->D, S = lb->S;
   const size_t DS = (size_t)D * S;
   hipStream_t st = lb->st;
-  Copies copies(lb);
+  Copies copies(lb, true);
   SEAMCHK(op, upload_cf(lb, lb->qkvt, 3 * D, q, D));
   SEAMCHK(op, upload_cf(lb, lb->qkvt + D, 3 * D, k, D));
   SEAMCHK(op, upload_cf(lb, lb->qkvt + 2 * D, 3 * D, v, D));

@@ -28,7 +28,7 @@ def engine(vocab, seed):
 # 64 floats a vocabulary row (and 128 KiB of layer weights): below the least
 # size of a copy through the pool, at it and past it, around one slot (4 MiB),
 # past the ring of 8 slots, past twice that
-@pytest.mark.parametrize("vocab", [256, 512, 1024, 15808, 15872, 16384, 131072 + 6400, 65536 * 4 + 64])
+@pytest.mark.parametrize("vocab", [256, 512, 1024, 3584, 3648, 15808, 15872, 16384, 131072 + 6400, 65536 * 4 + 64])
 def test_params_round_trip(vocab):
     other, _ = engine(40000, 3)  # (so that there is a pool, whatever this one's size)
     eng, p = engine(vocab, vocab)
