@@ -109,7 +109,7 @@ struct HostPoolRef {
 class HostCopy {
  public:
   // ref: the calling object's, filled by the copy from which the pool pays
-  // many: the call has eight copies or more
+  // many: the call has eight copies or more, or larger ones to come
   HostCopy(HostPoolRef* ref, int device, hipStream_t st, bool many = false)
       : ref_(ref), device_(device), st_(st), min_(many ? HostPool::kMoreBytes : HostPool::kMinBytes) {}
   ~HostCopy();

@@ -656,7 +656,9 @@ extern "C" int ane_layer_backward_run_ffn(ane_layer_bwd* lb, float* dx_norm, flo
   if (!dx_norm || !dh1 || !dffn || !h1) return seam_fail(ANE_ERR_ARG, "%s: null buffer", op);
   const int D = lb->D, H = lb->H, S = lb->S;
   hipStream_t st = lb->st;
-  Copies copies(lb);
+  // (where H S needs the pool, D S takes it too: the object's first copy by the
+  // runtime costs 300 us, for a staging buffer of its stream)
+  Copies copies(lb, (size_t)H * S * 4 >= HostPool::kMinBytes);
   SEAMCHK(op, upload_cf(lb, lb->dffn, D, dffn, D));
   SEAMCHK(op, upload_cf(lb, lb->h1, H, h1, H));
   {
