@@ -127,3 +127,24 @@ def test_a_tokens_loss_does_not_depend_on_its_neighbours(T):
     assert (lses[0][beside] != lses[2][beside]).all()
     for other in lses[1:]:
         np.testing.assert_array_equal(other[~beside], lses[0][~beside])
+
+
+def test_softcap_of_infinities_and_nan():
+    """+-infinity and the largest fp16 give +-cap exactly, NaN stays, and the
+    values beside them (of the same wave) are the softcap of themselves."""
+    lib = _lib.load()
+    M, N, K = 256, 64, 256
+    v = np.linspace(-4, 4, M).astype(np.float16)
+    v[[3, 40, 77, 130, 200]] = [np.inf, -np.inf, np.nan, 65504, -65504]
+    a = np.zeros((M, K), np.float16)
+    a[np.arange(M), np.arange(M)] = v
+    out = np.zeros((M, N), np.float32)
+    assert lib.ane_debug_gemm_epi(2, M, N, K, _u16(a), _u16(np.ones((N, K), np.float16)),
+                                  out.ctypes.data_as(C.c_void_p), None, None, None, 1.0, 0.0, -1, 0, 0,
+                                  0) == 0, lib.ane_debug_last_error()
+    for row, want in ((3, 15.0), (40, -15.0), (130, 15.0), (200, -15.0)):
+        assert (out[row] == want).all(), (row, out[row][:4])
+    assert np.isnan(out[77]).all()
+    rest = np.delete(np.arange(M), [3, 40, 77, 130, 200])
+    ref = 15.0 * np.tanh(v[rest].astype(np.float64) / 15.0)[:, None]
+    np.testing.assert_allclose(out[rest], np.broadcast_to(ref, (rest.size, N)), rtol=1.8e-7, atol=1e-30)
