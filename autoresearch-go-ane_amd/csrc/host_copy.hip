@@ -122,7 +122,9 @@ void HostPool::run() {
       asleep_.fetch_sub(1);
       if (stop_) return;
     }
-    cv_.notify_one();  // the next sleeper (the caller wakes one thread, not all: ~12 us each)
+    // the next two sleepers (the caller wakes one thread, not all: ~12 us each)
+    cv_.notify_one();
+    cv_.notify_one();
   }
 }
 
